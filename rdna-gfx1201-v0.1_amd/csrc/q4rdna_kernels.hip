@@ -732,21 +732,86 @@ __device__ GroupRange group_range(const float *v) {
 
 // The sidecar packer's sums at one scale, in fp32: the squared error of the
 // codes and the least-squares terms sum v*q and sum q*q of a refit.  One pass
-// computes all three from the same codes; each sum keeps index order.
+// computes all three from the same codes; each sum keeps index order.  Only
+// the groups and scales that fit_f32_quick leaves out come here (non-finite
+// values or scales, scale 0), so the values are read from memory again
+// instead of making 64 divisions' registers part of the common path.
 struct FitF32 {
     float err, num, den;
 };
 
-__device__ FitF32 fit_f32(const float *v, float s) {
+__device__ __forceinline__ FitF32 fit_f32(gptr_cf32 v, float s) {
     FitF32 f{0.0f, 0.0f, 0.0f};
+#pragma unroll 1
     for (int i = 0; i < 64; ++i) {
-        const int q = code_at<true>(v[i], s);
-        const float d = s * static_cast<float>(q) - v[i];
+        const float x = v[i];
+        const int q = code_at<true>(x, s);
+        const float d = s * static_cast<float>(q) - x;
         f.err += d * d;
-        f.num += v[i] * static_cast<float>(q);
+        f.num += x * static_cast<float>(q);
         f.den += static_cast<float>(q * q);
     }
     return f;
+}
+
+// fit_f32 without the divisions, for scales of the packer (fp16 values, so
+// at most 11 significant bits) that are finite and not zero and groups whose
+// values are finite and below 2^30 * |s|.  y is 1 / s, rounded.
+//
+// The code is rint(fl(v / s)) clamped to [-8, 7].  t = fma(v - s t0, y, t0)
+// with t0 = fl(v y) is v / s rounded once more from a value within
+// 2^-45 |v / s| of it: the residual v - s t0 is exact (s t0 has at most 35
+// bits, t0 is within 2 ulp of v / s).  Only the halves h = n + 1/2 below 8.5
+// decide a code.  s h has at most 16 bits, so either v = s h, and t = h
+// exactly, or v is off s h by at least one ulp of v, which puts v / s more
+// than (1 + 2^-11) half ulps of h away from h (the ulp below a power of two
+// is finer): then t and fl(v / s) lie on v's side of h, both.  So rint(t) is
+// the code, ties included.  s q is exact (15 bits), so fma(s, q, -v) is
+// fl(s q - v), and the sum of q q is a sum of small integers.
+__device__ __forceinline__ float quick_code(float v, float s, float y) {
+    const float t0 = v * y;
+    const float t = fmaf(fmaf(-s, t0, v), y, t0);
+    return __builtin_amdgcn_fmed3f(rintf(t), -8.0f, 7.0f);
+}
+
+__device__ __forceinline__ FitF32 fit_f32_quick(const float *v, float s) {
+    const float y = 1.0f / s;
+    FitF32 f{0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+        const float q = quick_code(v[i], s, y);
+        const float d = fmaf(s, q, -v[i]);
+        f.err += d * d;
+        f.num += v[i] * q;
+        f.den = fmaf(q, q, f.den);
+    }
+    return f;
+}
+
+// Whether fit_f32_quick and quick_code hold at scale s: `limit` is 2^-30 of
+// the group's largest magnitude, infinity for a group with non-finite values.
+__device__ __forceinline__ bool quick_scale(float s, float limit) { return fabsf(s) > limit && isfinite(s); }
+
+// The scales a lane has evaluated lately, as fp16 bits (0x7fff, a NaN the
+// packer never makes, marks an empty place).
+constexpr int kSeenScales = 8;
+struct SeenScales {
+    uint32_t pair[kSeenScales / 2];
+};
+__device__ __forceinline__ void seen_clear(SeenScales &m) {
+#pragma unroll
+    for (int i = 0; i < kSeenScales / 2; ++i) m.pair[i] = 0x7fff7fffu;
+}
+__device__ __forceinline__ void seen_add(SeenScales &m, uint32_t h) {
+#pragma unroll
+    for (int i = kSeenScales / 2 - 1; i > 0; --i) m.pair[i] = (m.pair[i] << 16) | (m.pair[i - 1] >> 16);
+    m.pair[0] = (m.pair[0] << 16) | h;
+}
+__device__ __forceinline__ bool seen(const SeenScales &m, uint32_t h) {
+    bool hit = false;
+#pragma unroll
+    for (int i = 0; i < kSeenScales / 2; ++i) hit |= (m.pair[i] & 0xffffu) == h || (m.pair[i] >> 16) == h;
+    return hit;
 }
 
 // Sidecar search: ten starts (the positive and the negative range scale,
@@ -754,27 +819,47 @@ __device__ FitF32 fit_f32(const float *v, float s) {
 // by least squares until its fp16 scale repeats, for at most 12 evaluations;
 // the scale of least error wins, the earliest on ties.  An all-zero group
 // gets scale 0.
-__device__ uint32_t search_sidecar(const float *v) {
-    const GroupRange g = group_range(v);
+//
+// A lane goes from one start to the next by itself (one loop over all its
+// evaluations), so a wave runs as long as its slowest lane in all and not
+// as the slowest lane of each start.  A start ends where it meets a scale
+// whose own evaluations have all been made: what follows a scale depends on
+// it alone, and an error met again is never strictly smaller.  A start cut
+// off by the limit of 12 leaves scales that do not qualify, so it empties
+// the memory.
+__device__ uint32_t search_sidecar(const float *v, gptr_cf32 src, const GroupRange &g, float limit) {
     if (g.pos_max == 0.0f && g.neg_max == 0.0f) return 0;
-    const float factor[5] = {1.0f, 0.9f, 0.8f, 0.7f, 0.6f};
     uint32_t best = 0;
     float best_err = __builtin_huge_valf();
-    for (int start = 0; start < 10; ++start) {
-        uint32_t h = packer_encode(((start & 1) ? g.neg_scale : g.pos_scale) * factor[start >> 1]);
-        for (int eval = 0; eval < 12; ++eval) {
-            const FitF32 f = fit_f32(v, packer_decode(h));
-            if (f.err < best_err) {
-                best_err = f.err;
-                best = h;
+    SeenScales met;
+    seen_clear(met);
+    int start = 0, eval = 0;
+    uint32_t h = packer_encode(g.pos_scale);
+    for (;;) {
+        const float s = packer_decode(h);
+        const FitF32 f = quick_scale(s, limit) ? fit_f32_quick(v, s) : fit_f32(src, s);
+        if (f.err < best_err) {
+            best_err = f.err;
+            best = h;
+        }
+        seen_add(met, h);
+        bool done = f.den == 0.0f;
+        if (!done) {
+            h = packer_encode(f.num / f.den);
+            done = seen(met, h);
+            if (++eval == 12 && !done) {
+                done = true;
+                seen_clear(met);
             }
-            if (f.den == 0.0f) break;
-            const uint32_t next = packer_encode(f.num / f.den);
-            if (next == h) break;
-            h = next;
+        }
+        while (done) {
+            if (++start == 10) return best;
+            eval = 0;
+            const float factor = start < 2 ? 1.0f : start < 4 ? 0.9f : start < 6 ? 0.8f : start < 8 ? 0.7f : 0.6f;
+            h = packer_encode(((start & 1) ? g.neg_scale : g.pos_scale) * factor);
+            done = seen(met, h);
         }
     }
-    return best;
 }
 
 // The CPU experiment's bookkeeping: the best fp16 scale so far and its
@@ -835,8 +920,7 @@ __device__ void refit_f64(const float *v, float s0, Best &b) {
 // The CPU experiment's three searches: absmax = fp16(max|v| / 7); range =
 // the better of the two range scales; mse = range, then 24 refitted starts
 // (the two range scales times 1 .. 0.25, positive first at each factor).
-__device__ uint32_t search_experiment(const float *v, int algorithm) {
-    const GroupRange g = group_range(v);
+__device__ uint32_t search_experiment(const float *v, const GroupRange &g, int algorithm) {
     if (g.abs_max == 0.0f) return 0;
     if (algorithm == 1) return packer_encode(g.abs_max / 7.0f);
     Best b{__builtin_huge_val(), 0u};
@@ -850,10 +934,12 @@ __device__ uint32_t search_experiment(const float *v, int algorithm) {
 }
 
 // Thread per (row, group) ordered (row tile, group, row lane) so a wave's
-// scale and code stores land in contiguous bytes of one tile.
-__global__ __launch_bounds__(kThreads) void pack_kernel(const float *__restrict__ w, uint32_t rows,
-                                                        uint32_t cols, int algorithm,
-                                                        uint8_t *__restrict__ tiles) {
+// scale and code stores land in contiguous bytes of one tile.  Bound by the
+// search's arithmetic.
+template <bool SIDECAR>
+__global__ __launch_bounds__(kThreads, SIDECAR ? 3 : 1) void pack_kernel(const float *__restrict__ w, uint32_t rows,
+                                                                         uint32_t cols, int algorithm,
+                                                                         uint8_t *__restrict__ tiles) {
     const uint32_t groups = cols / kGroup;
     const uint64_t total = static_cast<uint64_t>(rows) * groups;
     for (uint64_t idx = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; idx < total;
@@ -872,15 +958,42 @@ __global__ __launch_bounds__(kThreads) void pack_kernel(const float *__restrict_
             v[4 * i + 2] = f.z;
             v[4 * i + 3] = f.w;
         }
-        const uint32_t bits = algorithm == 0 ? search_sidecar(v) : search_experiment(v, algorithm);
-        const float scale = packer_decode(bits);
+        const GroupRange range = group_range(v);
         uint8_t *tile = tiles + t * kTileBytes;
-        tile[2 * l] = static_cast<uint8_t>(bits & 0xffu);
-        tile[2 * l + 1] = static_cast<uint8_t>(bits >> 8);
-        for (int i = 0; i < 32; ++i) {
-            const int lo = algorithm == 0 ? code_at<true>(v[2 * i], scale) : code_at<false>(v[2 * i], scale);
-            const int hi = algorithm == 0 ? code_at<true>(v[2 * i + 1], scale) : code_at<false>(v[2 * i + 1], scale);
-            tile[64 + 32 * i + l] = static_cast<uint8_t>((lo & 15) | ((hi & 15) << 4));
+        if constexpr (SIDECAR) {
+            bool finite = true;
+#pragma unroll
+            for (int i = 0; i < 64; ++i) finite &= isfinite(v[i]);
+            const float limit = finite ? range.abs_max * 0x1p-30f : __builtin_huge_valf();
+            const uint32_t bits = search_sidecar(v, (gptr_cf32)src, range, limit);
+            const float scale = packer_decode(bits);
+            tile[2 * l] = static_cast<uint8_t>(bits & 0xffu);
+            tile[2 * l + 1] = static_cast<uint8_t>(bits >> 8);
+            if (quick_scale(scale, limit)) {
+                const float y = 1.0f / scale;
+#pragma unroll
+                for (int i = 0; i < 32; ++i) {
+                    const int lo = static_cast<int>(quick_code(v[2 * i], scale, y));
+                    const int hi = static_cast<int>(quick_code(v[2 * i + 1], scale, y));
+                    tile[64 + 32 * i + l] = static_cast<uint8_t>((lo & 15) | ((hi & 15) << 4));
+                }
+            } else {
+                const gptr_cf32 x = (gptr_cf32)src;
+#pragma unroll 1
+                for (int i = 0; i < 32; ++i) {
+                    const int lo = code_at<true>(x[2 * i], scale), hi = code_at<true>(x[2 * i + 1], scale);
+                    tile[64 + 32 * i + l] = static_cast<uint8_t>((lo & 15) | ((hi & 15) << 4));
+                }
+            }
+        } else {
+            const uint32_t bits = search_experiment(v, range, algorithm);
+            const float scale = packer_decode(bits);
+            tile[2 * l] = static_cast<uint8_t>(bits & 0xffu);
+            tile[2 * l + 1] = static_cast<uint8_t>(bits >> 8);
+            for (int i = 0; i < 32; ++i) {
+                const int lo = code_at<false>(v[2 * i], scale), hi = code_at<false>(v[2 * i + 1], scale);
+                tile[64 + 32 * i + l] = static_cast<uint8_t>((lo & 15) | ((hi & 15) << 4));
+            }
         }
     }
 }
@@ -1047,8 +1160,11 @@ hipError_t launch_dequant(const uint8_t *w, uint32_t rows, uint32_t cols, float 
 hipError_t launch_pack(const float *w, uint32_t rows, uint32_t cols, int algorithm, uint8_t *tiles,
                        hipStream_t stream) {
     const uint64_t work = static_cast<uint64_t>(rows) * (cols / kGroup);
-    hipLaunchKernelGGL(pack_kernel, dim3(grid_for(work, kThreads)), dim3(kThreads), 0, stream, w, rows, cols,
-                       algorithm, tiles);
+    const dim3 grid(grid_for(work, kThreads)), block(kThreads);
+    if (algorithm == 0)
+        hipLaunchKernelGGL(pack_kernel<true>, grid, block, 0, stream, w, rows, cols, algorithm, tiles);
+    else
+        hipLaunchKernelGGL(pack_kernel<false>, grid, block, 0, stream, w, rows, cols, algorithm, tiles);
     return hipGetLastError();
 }
 
