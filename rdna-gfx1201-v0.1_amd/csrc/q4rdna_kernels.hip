@@ -754,32 +754,38 @@ __device__ __forceinline__ FitF32 fit_f32(gptr_cf32 v, float s) {
     return f;
 }
 
+// 1 / s as an unevaluated sum, within 2^-47 of it (relatively).
+struct Reciprocal {
+    float hi, lo;
+};
+__device__ __forceinline__ Reciprocal reciprocal(float s) {
+    const float y = 1.0f / s;
+    return Reciprocal{y, fmaf(-s, y, 1.0f) * y};
+}
+
 // fit_f32 without the divisions, for scales of the packer (fp16 values, so
 // at most 11 significant bits) that are finite and not zero and groups whose
-// values are finite and below 2^30 * |s|.  y is 1 / s, rounded.
+// values are finite and below 2^30 * |s|.
 //
-// The code is rint(fl(v / s)) clamped to [-8, 7].  t = fma(v - s t0, y, t0)
-// with t0 = fl(v y) is v / s rounded once more from a value within
-// 2^-45 |v / s| of it: the residual v - s t0 is exact (s t0 has at most 35
-// bits, t0 is within 2 ulp of v / s).  Only the halves h = n + 1/2 below 8.5
-// decide a code.  s h has at most 16 bits, so either v = s h, and t = h
-// exactly, or v is off s h by at least one ulp of v, which puts v / s more
-// than (1 + 2^-11) half ulps of h away from h (the ulp below a power of two
-// is finer): then t and fl(v / s) lie on v's side of h, both.  So rint(t) is
-// the code, ties included.  s q is exact (15 bits), so fma(s, q, -v) is
-// fl(s q - v), and the sum of q q is a sum of small integers.
-__device__ __forceinline__ float quick_code(float v, float s, float y) {
-    const float t0 = v * y;
-    const float t = fmaf(fmaf(-s, t0, v), y, t0);
-    return __builtin_amdgcn_fmed3f(rintf(t), -8.0f, 7.0f);
+// The code is rint(fl(v / s)) clamped to [-8, 7].  t = fma(v, y.hi, v y.lo)
+// is v / s rounded once from a value within 2^-46 |v / s| of it.  Only the
+// halves h = n + 1/2 below 8.5 decide a code.  s h has at most 16 bits, so
+// either v = s h, and t = h exactly, or v is off s h by at least one ulp of
+// v, which puts v / s more than (1 + 2^-11) half ulps of h away from h (the
+// ulp below a power of two is finer): then t and fl(v / s) lie on v's side
+// of h, both.  So rint(t) is the code, ties included.  s q is exact (15
+// bits), so fma(s, q, -v) is fl(s q - v), and the sum of q q is a sum of
+// small integers.
+__device__ __forceinline__ float quick_code(float v, Reciprocal y) {
+    return __builtin_amdgcn_fmed3f(rintf(fmaf(v, y.hi, v * y.lo)), -8.0f, 7.0f);
 }
 
 __device__ __forceinline__ FitF32 fit_f32_quick(const float *v, float s) {
-    const float y = 1.0f / s;
+    const Reciprocal y = reciprocal(s);
     FitF32 f{0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
-        const float q = quick_code(v[i], s, y);
+        const float q = quick_code(v[i], y);
         const float d = fmaf(s, q, -v[i]);
         f.err += d * d;
         f.num += v[i] * q;
@@ -792,26 +798,20 @@ __device__ __forceinline__ FitF32 fit_f32_quick(const float *v, float s) {
 // the group's largest magnitude, infinity for a group with non-finite values.
 __device__ __forceinline__ bool quick_scale(float s, float limit) { return fabsf(s) > limit && isfinite(s); }
 
-// The scales a lane has evaluated lately, as fp16 bits (0x7fff, a NaN the
-// packer never makes, marks an empty place).
-constexpr int kSeenScales = 8;
+// The scales a thread has evaluated: fp16 bits h in place h % kSeenScales of
+// its column, the latest of that place (0x7fff, a NaN the packer never makes,
+// marks an empty place; forgetting a scale only costs evaluating it again).
+// With 64 places a Gaussian group makes 48 evaluations instead of 65 and a
+// wave, which runs as long as its slowest lane, 66 instead of 88.
+constexpr int kSeenScales = 64;
 struct SeenScales {
-    uint32_t pair[kSeenScales / 2];
+    uint16_t h[kSeenScales][kThreads];
 };
 __device__ __forceinline__ void seen_clear(SeenScales &m) {
-#pragma unroll
-    for (int i = 0; i < kSeenScales / 2; ++i) m.pair[i] = 0x7fff7fffu;
-}
-__device__ __forceinline__ void seen_add(SeenScales &m, uint32_t h) {
-#pragma unroll
-    for (int i = kSeenScales / 2 - 1; i > 0; --i) m.pair[i] = (m.pair[i] << 16) | (m.pair[i - 1] >> 16);
-    m.pair[0] = (m.pair[0] << 16) | h;
+    for (int i = 0; i < kSeenScales; ++i) m.h[i][threadIdx.x] = 0x7fff;
 }
 __device__ __forceinline__ bool seen(const SeenScales &m, uint32_t h) {
-    bool hit = false;
-#pragma unroll
-    for (int i = 0; i < kSeenScales / 2; ++i) hit |= (m.pair[i] & 0xffffu) == h || (m.pair[i] >> 16) == h;
-    return hit;
+    return m.h[h % kSeenScales][threadIdx.x] == h;
 }
 
 // Sidecar search: ten starts (the positive and the negative range scale,
@@ -827,11 +827,10 @@ __device__ __forceinline__ bool seen(const SeenScales &m, uint32_t h) {
 // it alone, and an error met again is never strictly smaller.  A start cut
 // off by the limit of 12 leaves scales that do not qualify, so it empties
 // the memory.
-__device__ uint32_t search_sidecar(const float *v, gptr_cf32 src, const GroupRange &g, float limit) {
+__device__ uint32_t search_sidecar(const float *v, gptr_cf32 src, const GroupRange &g, float limit, SeenScales &met) {
     if (g.pos_max == 0.0f && g.neg_max == 0.0f) return 0;
     uint32_t best = 0;
     float best_err = __builtin_huge_valf();
-    SeenScales met;
     seen_clear(met);
     int start = 0, eval = 0;
     uint32_t h = packer_encode(g.pos_scale);
@@ -842,7 +841,7 @@ __device__ uint32_t search_sidecar(const float *v, gptr_cf32 src, const GroupRan
             best_err = f.err;
             best = h;
         }
-        seen_add(met, h);
+        met.h[h % kSeenScales][threadIdx.x] = static_cast<uint16_t>(h);
         bool done = f.den == 0.0f;
         if (!done) {
             h = packer_encode(f.num / f.den);
@@ -935,7 +934,10 @@ __device__ uint32_t search_experiment(const float *v, const GroupRange &g, int a
 
 // Thread per (row, group) ordered (row tile, group, row lane) so a wave's
 // scale and code stores land in contiguous bytes of one tile.  Bound by the
-// search's arithmetic.
+// search's arithmetic, ten VALU operations per value and evaluation:
+// 12288x4096 takes 836 us, with a division per value and evaluation and the
+// starts in step it took 6257 us.  Three waves per SIMD are what the group's
+// 64 values and the working set leave; a limit of four spills.
 template <bool SIDECAR>
 __global__ __launch_bounds__(kThreads, SIDECAR ? 3 : 1) void pack_kernel(const float *__restrict__ w, uint32_t rows,
                                                                          uint32_t cols, int algorithm,
@@ -961,20 +963,21 @@ __global__ __launch_bounds__(kThreads, SIDECAR ? 3 : 1) void pack_kernel(const f
         const GroupRange range = group_range(v);
         uint8_t *tile = tiles + t * kTileBytes;
         if constexpr (SIDECAR) {
+            __shared__ SeenScales met;
             bool finite = true;
 #pragma unroll
             for (int i = 0; i < 64; ++i) finite &= isfinite(v[i]);
             const float limit = finite ? range.abs_max * 0x1p-30f : __builtin_huge_valf();
-            const uint32_t bits = search_sidecar(v, (gptr_cf32)src, range, limit);
+            const uint32_t bits = search_sidecar(v, (gptr_cf32)src, range, limit, met);
             const float scale = packer_decode(bits);
             tile[2 * l] = static_cast<uint8_t>(bits & 0xffu);
             tile[2 * l + 1] = static_cast<uint8_t>(bits >> 8);
             if (quick_scale(scale, limit)) {
-                const float y = 1.0f / scale;
+                const Reciprocal y = reciprocal(scale);
 #pragma unroll
                 for (int i = 0; i < 32; ++i) {
-                    const int lo = static_cast<int>(quick_code(v[2 * i], scale, y));
-                    const int hi = static_cast<int>(quick_code(v[2 * i + 1], scale, y));
+                    const int lo = static_cast<int>(quick_code(v[2 * i], y));
+                    const int hi = static_cast<int>(quick_code(v[2 * i + 1], y));
                     tile[64 + 32 * i + l] = static_cast<uint8_t>((lo & 15) | ((hi & 15) << 4));
                 }
             } else {
