@@ -936,8 +936,6 @@ __device__ uint32_t search_experiment(const float *v, const GroupRange &g, int a
 // scale and code stores land in contiguous bytes of one tile.  Bound by the
 // search's arithmetic, ten VALU operations per value and evaluation:
 // 12288x4096 takes 836 us, with a division per value and evaluation and the
-// starts in step it took 6257 us.  Three waves per SIMD are what the group's
-// 64 values and the working set leave; a limit of four spills.
 template <bool SIDECAR>
 __global__ __launch_bounds__(kThreads, SIDECAR ? 3 : 1) void pack_kernel(const float *__restrict__ w, uint32_t rows,
                                                                          uint32_t cols, int algorithm,
