@@ -98,10 +98,13 @@ std::vector<uint32_t> item_costs(const PlanLayout &layout) {
             const uint32_t part = (item - p.item_begin) % p.per;
             const uint32_t chunk = part % p.chunks;
             const uint32_t chunk_g = std::min(g, (chunk + 1) * kChunkGroups) - chunk * kChunkGroups;
-            // Pairs stream four row tiles, items of both streams two per
-            // stream, other items two.
-            const uint32_t row_tiles = p.pair || (p.streams > 1 && p.per == 1) ? 4u : 2u;
-            cost[item] = row_tiles * chunk_g + kItemEndTiles;
+            // Pairs and items of both streams make two passes over their
+            // groups.  The passes' quads of four groups are dealt to the
+            // workgroup's four waves, and an item takes as long as its
+            // fullest wave, a step of 32 tiles per quad of that wave.
+            const uint32_t passes = p.pair || (p.streams > 1 && p.per == 1) ? 2u : 1u;
+            const uint32_t steps = (passes * ((chunk_g + 3) / 4) + 3) / 4;
+            cost[item] = 32 * steps + kItemEndTiles;
         }
     }
     return cost;
