@@ -89,6 +89,12 @@ uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus) {
     return std::max<uint32_t>(split, 1);
 }
 
+// Steps of 32 tiles of a single-vector item: pairs and items of both streams
+// make two passes over their groups, the passes' quads of four groups are
+// dealt to the workgroup's four waves, and the item takes as long as its
+// fullest wave.
+static uint32_t item_steps(uint32_t groups, uint32_t passes) { return (passes * ((groups + 3) / 4) + 3) / 4; }
+
 std::vector<uint32_t> item_costs(const PlanLayout &layout) {
     std::vector<uint32_t> cost(layout.items);
     for (uint32_t i = 0; i < layout.count; ++i) {
@@ -98,13 +104,8 @@ std::vector<uint32_t> item_costs(const PlanLayout &layout) {
             const uint32_t part = (item - p.item_begin) % p.per;
             const uint32_t chunk = part % p.chunks;
             const uint32_t chunk_g = std::min(g, (chunk + 1) * kChunkGroups) - chunk * kChunkGroups;
-            // Pairs and items of both streams make two passes over their
-            // groups.  The passes' quads of four groups are dealt to the
-            // workgroup's four waves, and an item takes as long as its
-            // fullest wave, a step of 32 tiles per quad of that wave.
             const uint32_t passes = p.pair || (p.streams > 1 && p.per == 1) ? 2u : 1u;
-            const uint32_t steps = (passes * ((chunk_g + 3) / 4) + 3) / 4;
-            cost[item] = 32 * steps + kItemEndTiles;
+            cost[item] = 32 * item_steps(chunk_g, passes) + kItemEndTiles;
         }
     }
     return cost;
@@ -300,15 +301,34 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     // end of the sweep, where workgroups run out of items, deals short ones.
     L.order.resize(count);
     for (uint32_t i = 0; i < count; ++i) L.order[i] = i;
+    // Single-vector items are as large as the plan's work allows: `share` is
+    // the steps of a workgroup if all ran the same number.
+    const uint64_t workgroups = uint64_t(cus) * kPlanWorkgroupsPerCu;
+    uint64_t steps = 0;
+    for (uint32_t i = 0; i < count; ++i)
+        steps += static_cast<uint64_t>((descs[i].weight.rows + block_rows - 1) / block_rows) *
+                 item_steps(descs[i].weight.columns / kGroup, descs[i].gate_tiles != nullptr ? 2 : 1);
+    const double share = static_cast<double>(steps) / static_cast<double>(workgroups);
     // A SwiGLU GEMV whose rows fit one chunk runs both weight streams in one
     // item per block (no split-K partials), single vectors and batches alike.
+    // That saves the two streams' meeting in memory, about two steps' time;
+    // beyond twice the share the item costs more than that (the other
+    // workgroups are done before it) and the streams are items of their own.
     auto both_streams = [&](uint32_t i) {
-        return descs[i].gate_tiles != nullptr && descs[i].weight.columns / kGroup <= chunk_groups;
+        const uint32_t g = descs[i].weight.columns / kGroup;
+        return descs[i].gate_tiles != nullptr && g <= chunk_groups && (n > 1 || item_steps(g, 2) <= 2.0 * share);
     };
     // A single-vector GEMV with no gate whose rows fit one 64-group step
-    // block runs two 64-row blocks per item: half the item ends.
+    // block runs two 64-row blocks per item: half the item ends.  One block
+    // costs nothing else, so two are taken only up to half a share: two
+    // Qwen3-8B layers (share 11.5 steps) run in 37.4 us instead of 42.6, eight
+    // layers of 1024 and 2816 columns (share 2.7) in 14.7 instead of 17.1; at
+    // four Qwen3-8B layers both measure 67.8.
     auto pairs = [&](uint32_t i) {
-        return n == 1 && descs[i].gate_tiles == nullptr && descs[i].weight.columns / kGroup <= 64;
+        const uint32_t g = descs[i].weight.columns / kGroup;
+        const uint32_t pair_steps = item_steps(g, 2);
+        return n == 1 && descs[i].gate_tiles == nullptr && g <= kPairGroups &&
+               (pair_steps <= 1 || pair_steps <= 0.5 * share);
     };
     auto item_groups = [&](uint32_t i) {
         return std::min(descs[i].weight.columns / kGroup, chunk_groups) * (both_streams(i) || pairs(i) ? 2u : 1u);

@@ -62,8 +62,8 @@ struct GemvArgs {
 // (64-row block, stream, K chunk of up to kChunkGroups groups), numbered from
 // item_begin block-major, then stream (0 = w, 1 = the SwiGLU gate), then
 // chunk; `per` items per block.  A single-vector SwiGLU GEMV whose rows fit
-// one chunk has per = 1: its item streams both weights.  A `pair` GEMV
-// (single vector, no gate, rows of at most 64 groups) has items of two
+// one chunk may have per = 1: its item streams both weights.  A `pair` GEMV
+// (single vector, no gate, rows of at most kPairGroups groups) has items of two
 // 64-row blocks, numbered from item_begin, one per 128 rows.  The activation is
 // first converted into int8 digits (kPrepBytes per 64-element group) in
 // `prep`.  When a block has more than one item (per > 1) its items meet in
@@ -119,6 +119,8 @@ constexpr uint32_t kGemvClockWords = 6;  // start, staged, reduced, end, HW_ID, 
 // K chunk of a single-vector plan item: 192 groups holds a whole 12288-wide
 // row in one item, so such GEMVs need no split-K partials.
 constexpr uint32_t kChunkGroups = 192;
+// Longest rows that pair items take.
+constexpr uint32_t kPairGroups = 64;
 constexpr uint32_t kBlockRows = 64;
 
 // The kernels divide by the split with a multiply: magic = ceil(2^32 /

@@ -693,6 +693,7 @@ struct ItemCtx {
     const uint8_t *rt[4];
     const uint8_t *prep;
     uint32_t g_begin, g_end, kind;
+    uint32_t first;  // quads dealt to the waves before this item's
     ItemOut o;
 };
 
@@ -710,6 +711,7 @@ __device__ __forceinline__ ItemCtx decode_item(const PlanDesc &d, uint32_t local
         for (int i = 0; i < 4; ++i) c.rt[i] = d.w + static_cast<size_t>(min(4 * local + i, tiles - 1)) * row_tile_bytes;
         c.g_begin = 0;
         c.g_end = groups;
+        c.first = 0;
         c.kind = kPairPass;
         c.o = ItemOut{d.add, d.y, nullptr, nullptr, d.rows, local, 0, 1, 1, 1};
         return c;
@@ -720,6 +722,11 @@ __device__ __forceinline__ ItemCtx decode_item(const PlanDesc &d, uint32_t local
     const uint32_t stream = both ? 0 : part / d.chunks, chunk = both ? 0 : part - stream * d.chunks;
     c.g_begin = chunk * kChunkGroups;
     c.g_end = min(groups, c.g_begin + kChunkGroups);
+    // Where two-pass items would run this part as their second pass, its
+    // quads go to the same waves: a row's sums do not depend on whether the
+    // plan took the larger or the smaller item.
+    const bool second_pass = stream != 0 || (d.streams == 1 && groups <= kPairGroups && (block & 1u) != 0u);
+    c.first = second_pass ? (c.g_end - c.g_begin + kStepGroups - 1) / kStepGroups : 0;
     // The second row tile of a block past the last one re-reads the last
     // (its rows are never written).
     const size_t block_offset = static_cast<size_t>(2 * block) * row_tile_bytes;
@@ -771,8 +778,8 @@ __global__ __launch_bounds__(256) void plan_kernel(const PlanDesc *__restrict__ 
         float acc[16], acc1[16];
 #pragma unroll
         for (int n = 0; n < 16; ++n) acc[n] = acc1[n] = 0.0f;
-        const uint32_t q = item_steps(cur.rt[0], cur.rt[1], cur.prep, cur.g_begin, cur.g_end, wave, lane, ln,
-                                      sh.stage[wave], acc, pre, have_pre);
+        const uint32_t q = item_steps(cur.rt[0], cur.rt[1], cur.prep, cur.g_begin, cur.g_end,
+                                      (wave - cur.first) % kWaves, lane, ln, sh.stage[wave], acc, pre, have_pre);
         if (cur.kind != kOnePass)
             item_steps(cur.rt[2], cur.rt[3], cur.prep, cur.g_begin, cur.g_end, q, lane, ln, sh.stage[wave], acc1, pre,
                        false);
@@ -781,8 +788,9 @@ __global__ __launch_bounds__(256) void plan_kernel(const PlanDesc *__restrict__ 
         have_pre = false;
         if (k < end) {
             next = locate(next_entry);
-            if (kStepGroups * (static_cast<uint32_t>(wave) + 1) <= next.g_end - next.g_begin) {
-                const uint32_t g = next.g_begin + kStepGroups * wave;
+            const uint32_t nq = (wave - next.first) % kWaves;
+            if (kStepGroups * (nq + 1) <= next.g_end - next.g_begin) {
+                const uint32_t g = next.g_begin + kStepGroups * nq;
                 load_step_regs(pre, next.rt[0] + static_cast<size_t>(g) * kTileBytes,
                                next.rt[1] + static_cast<size_t>(g) * kTileBytes, next.prep, g, ln, lane);
                 have_pre = true;

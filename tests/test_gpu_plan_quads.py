@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("groups", [[1, 2, 3, 4], [5, 7, 8, 9, 11], [13, 15, 16, 17, 24], [41, 63, 64, 65, 193, 195]])
 @pytest.mark.parametrize("kind", ["plain", "add", "glu"])
-def test_plan_uneven_groups(cuda, groups, kind):
+@pytest.mark.parametrize("repeat", [0, 60])
+def test_plan_uneven_groups(cuda, groups, kind, repeat):
     items, want = [], []
     for i, g in enumerate(groups):
         rows, cols = (32, 96, 160, 192, 320)[i % 5], 64 * g
@@ -28,9 +29,8 @@ def test_plan_uneven_groups(cuda, groups, kind):
                       None if gate_t is None else api.QWeight.from_tiles(dev_u8(gate_t), rows, cols),
                       None if add is None else dev_f32(add)))
         want.append((tiles, rows, cols, x, gate_t, add))
-    # Enough copies of the GEMVs that workgroups run several items each.
     copies = []
-    for _ in range(60):
+    for _ in range(repeat):
         for w, x, y, gate, add in items:
             copies.append((w, x, torch.full_like(y, float("nan")), gate, add))
     plan = api.Plan(items + copies)
@@ -40,4 +40,12 @@ def test_plan_uneven_groups(cuda, groups, kind):
         assert_gemv_parity(y.cpu().numpy(), tiles, rows, cols, x, gate_tiles=gate_t, add=add, label=(kind, cols))
     for i, c in enumerate(copies):
         assert torch.equal(c[2], items[i % len(items)][2]), i
+    plan.close()
+    # Alone, a GEMV runs the smaller items: the same bits.
+    w, x, y, gate, add = items[-1]
+    alone = torch.full_like(y, float("nan"))
+    plan = api.Plan([(w, x, alone, gate, add)])
+    assert plan.launch()
+    torch.cuda.synchronize()
+    assert torch.equal(alone, y)
     plan.close()
