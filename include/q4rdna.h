@@ -261,16 +261,20 @@ typedef struct q4rdna_gemv_desc {
 typedef struct q4rdna_plan q4rdna_plan;
 
 /* Build a plan for `count` descriptors (uploads the descriptor table once).
- * Single-vector plans also fix here which workgroup runs which item: a
- * load-balancing deal computed on the host, about 2 ms for the 252-tensor
- * Qwen3-8B stack and 0.2 s for 100,000 items. */
+ * Plans also fix here which workgroup runs which item: a load-balancing deal
+ * computed on the host, about 2 ms for the 252-tensor Qwen3-8B stack and
+ * 0.2 s for 100,000 items. */
 int q4rdna_plan_create(const q4rdna_gemv_desc *descs, uint32_t count, int device,
                        q4rdna_plan **out);
 /* Batched plan: every descriptor's x holds n activation vectors of
  * `columns` floats one after another ([n][columns]), y and add hold n
  * results of `rows` floats ([n][rows]); n = 1..Q4RDNA_MAX_BATCH (the
- * small-batch decode shapes).  No reference counterpart: the reference's
- * hooks decline batches above 1 (source/q4rdna.cu:722,754,777). */
+ * small-batch decode shapes).  A plan with little work per workgroup cuts
+ * long rows into more K chunks, so the order of a row's sum, and with it the
+ * last bits, depends on the shapes in the plan (not on n, the values or the
+ * order of the descriptors; a single-vector plan's sums depend on their own
+ * shape alone).  No reference counterpart: the reference's hooks decline
+ * batches above 1 (source/q4rdna.cu:722,754,777). */
 #define Q4RDNA_MAX_BATCH 8
 int q4rdna_plan_create_batch(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int device,
                              q4rdna_plan **out);

@@ -89,11 +89,15 @@ uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus) {
     return std::max<uint32_t>(split, 1);
 }
 
-// Steps of 32 tiles of a single-vector item: pairs and items of both streams
-// make two passes over their groups, the passes' quads of four groups are
-// dealt to the workgroup's four waves, and the item takes as long as its
-// fullest wave.
-static uint32_t item_steps(uint32_t groups, uint32_t passes) { return (passes * ((groups + 3) / 4) + 3) / 4; }
+// Steps of 32 tiles of an item that makes `passes` passes over its groups.
+// Single vectors: a step of a wave is a quad of four groups by two row tiles,
+// the passes' quads are dealt to the workgroup's four waves, and the item
+// takes as long as its fullest wave.  Batches: a wave's step is one group by
+// eight row tiles, each pass's groups dealt from the first wave on.
+static uint32_t steps_of(uint32_t batch, uint32_t groups, uint32_t passes) {
+    const uint32_t quads = (groups + 3) / 4;
+    return batch == 1 ? (passes * quads + 3) / 4 : passes * quads;
+}
 
 std::vector<uint32_t> item_costs(const PlanLayout &layout) {
     std::vector<uint32_t> cost(layout.items);
@@ -103,9 +107,10 @@ std::vector<uint32_t> item_costs(const PlanLayout &layout) {
         for (uint32_t item = p.item_begin; item < layout.descs[i + 1].item_begin; ++item) {
             const uint32_t part = (item - p.item_begin) % p.per;
             const uint32_t chunk = part % p.chunks;
-            const uint32_t chunk_g = std::min(g, (chunk + 1) * kChunkGroups) - chunk * kChunkGroups;
+            const uint32_t chunk_g = std::min(g, (chunk + 1) * p.chunk_groups) - chunk * p.chunk_groups;
             const uint32_t passes = p.pair || (p.streams > 1 && p.per == 1) ? 2u : 1u;
-            cost[item] = 32 * item_steps(chunk_g, passes) + kItemEndTiles;
+            cost[item] = 32 * steps_of(layout.batch, chunk_g, passes) +
+                         (layout.batch == 1 ? kItemEndTiles : kBatchItemEndTiles);
         }
     }
     return cost;
@@ -227,6 +232,14 @@ std::vector<uint32_t> deal_items(const std::vector<uint32_t> &cost, const std::v
     return deal;
 }
 
+// Whether a batched sweep claims its items from a queue.  The fixed deal lets
+// the next item's loads cross an item's end, which counts while a workgroup
+// runs few items; over many, up to four vectors gain more from the balance:
+// at N = 2 the 36 layers of Qwen3-8B (share 207 steps) take 620 us with the
+// deal and 598 with the queue, 18 layers 315 and 331, 9 layers 174 and 202.
+// With eight vectors the deal is ahead throughout (667 against 687 us).
+static bool batch_queue(uint32_t n, double share) { return n > 1 && n <= 4 && share > 140.0; }
+
 int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int device, uint32_t cus, PlanLayout *out,
                 std::string *error) {
     if (out == nullptr || (descs == nullptr && count > 0))
@@ -301,14 +314,31 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     // end of the sweep, where workgroups run out of items, deals short ones.
     L.order.resize(count);
     for (uint32_t i = 0; i < count; ++i) L.order[i] = i;
-    // Single-vector items are as large as the plan's work allows: `share` is
-    // the steps of a workgroup if all ran the same number.
+    // Items are as large as the plan's work allows: `share` is the steps of a
+    // workgroup if all ran the same number.
     const uint64_t workgroups = uint64_t(cus) * kPlanWorkgroupsPerCu;
     uint64_t steps = 0;
     for (uint32_t i = 0; i < count; ++i)
         steps += static_cast<uint64_t>((descs[i].weight.rows + block_rows - 1) / block_rows) *
-                 item_steps(descs[i].weight.columns / kGroup, descs[i].gate_tiles != nullptr ? 2 : 1);
+                 steps_of(n, descs[i].weight.columns / kGroup, descs[i].gate_tiles != nullptr ? 2 : 1);
     const double share = static_cast<double>(steps) / static_cast<double>(workgroups);
+    // Items well beyond a share are cut (a SwiGLU site into its streams; a
+    // batch's rows also into K chunks of about a share): the other workgroups
+    // are done before them, which costs more than the parts' meeting in
+    // memory.  Batches, us per step at N = 2 / 8, whole items against these:
+    // one Qwen3-8B layer (share 5.8) 78 / 94 against 33 / 44, four (share 23)
+    // 104 / 105 against 88 / 96; cutting from 1.25 shares on took 118 instead
+    // of 115 at an eighth of Qwen3-8B's widths (share 26) and N = 8.  A single
+    // vector's K chunks are not cut: its sums do not depend on the plan.
+    auto too_long = [&](uint32_t item) { return item > (n == 1 ? 2.0 : 1.6) * share; };
+    auto chunk_of = [&](uint32_t i) {
+        const uint32_t g = descs[i].weight.columns / kGroup;
+        if (n == 1 || !too_long(steps_of(n, std::min(g, chunk_groups), 1))) return chunk_groups;
+        const uint32_t least = share < 2.0 ? kMinBatchChunkGroups / 2 : kMinBatchChunkGroups;
+        const uint32_t most = std::min(chunk_groups, std::max(least, 4 * static_cast<uint32_t>(share)));
+        const uint32_t chunks = (g + most - 1) / most;
+        return ((g + chunks - 1) / chunks + 3) / 4 * 4;
+    };
     // A SwiGLU GEMV whose rows fit one chunk runs both weight streams in one
     // item per block (no split-K partials), single vectors and batches alike.
     // That saves the two streams' meeting in memory, about two steps' time;
@@ -316,7 +346,7 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     // workgroups are done before it) and the streams are items of their own.
     auto both_streams = [&](uint32_t i) {
         const uint32_t g = descs[i].weight.columns / kGroup;
-        return descs[i].gate_tiles != nullptr && g <= chunk_groups && (n > 1 || item_steps(g, 2) <= 2.0 * share);
+        return descs[i].gate_tiles != nullptr && g <= chunk_of(i) && !too_long(steps_of(n, g, 2));
     };
     // A single-vector GEMV with no gate whose rows fit one 64-group step
     // block runs two 64-row blocks per item: half the item ends.  One block
@@ -326,12 +356,12 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     // four Qwen3-8B layers both measure 67.8.
     auto pairs = [&](uint32_t i) {
         const uint32_t g = descs[i].weight.columns / kGroup;
-        const uint32_t pair_steps = item_steps(g, 2);
+        const uint32_t pair_steps = steps_of(n, g, 2);
         return n == 1 && descs[i].gate_tiles == nullptr && g <= kPairGroups &&
                (pair_steps <= 1 || pair_steps <= 0.5 * share);
     };
     auto item_groups = [&](uint32_t i) {
-        return std::min(descs[i].weight.columns / kGroup, chunk_groups) * (both_streams(i) || pairs(i) ? 2u : 1u);
+        return std::min(descs[i].weight.columns / kGroup, chunk_of(i)) * (both_streams(i) || pairs(i) ? 2u : 1u);
     };
     std::stable_sort(L.order.begin(), L.order.end(),
                      [&](uint32_t a, uint32_t b) { return item_groups(a) > item_groups(b); });
@@ -343,7 +373,8 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     for (uint32_t i = 0; i < count; ++i) {
         const q4rdna_gemv_desc &d = descs[L.order[i]];
         const uint32_t g = d.weight.columns / kGroup;
-        const uint32_t chunks = (g + chunk_groups - 1) / chunk_groups;
+        const uint32_t chunk = chunk_of(L.order[i]);
+        const uint32_t chunks = (g + chunk - 1) / chunk;
         const bool pair = pairs(L.order[i]);
         const uint32_t item_rows = pair ? 2 * block_rows : block_rows;
         const uint32_t blocks = (d.weight.rows + item_rows - 1) / item_rows;
@@ -362,6 +393,7 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
         p.streams = streams;
         p.per = both_streams(L.order[i]) || pair ? 1u : chunks * streams;
         p.pair = pair ? 1u : 0u;
+        p.chunk_groups = chunk;
         L.prep_off[i] = groups * prep_per_group;
         if (p.per > 1) {
             L.part_off[i] = tail;
@@ -387,25 +419,31 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     L.table_bytes = groups * (n == 1 ? sizeof(uint64_t) : sizeof(uint32_t));
     L.workgroups = static_cast<uint32_t>(
         std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(cus) * kPlanWorkgroupsPerCu, items)));
-    // Single vectors: the items' deal to the workgroups, after the table, in
-    // the kernel's form: the offsets (padded to an even count), then per item
-    // its descriptor index and its index within the descriptor.
-    if (n == 1) {
+    // After the group table, the items' list: per item its descriptor index
+    // and its index within the descriptor, in item order for a queue; as
+    // dealt to the workgroups, behind the deal's offsets (padded to an even
+    // count), otherwise.
+    std::vector<uint32_t> owner(items);
+    for (uint32_t i = 0; i < count; ++i)
+        for (uint32_t item = L.descs[i].item_begin; item < L.descs[i + 1].item_begin; ++item) owner[item] = i;
+    auto entry = [&](uint32_t *out, uint32_t item) {
+        out[0] = owner[item];
+        out[1] = item - L.descs[owner[item]].item_begin;
+    };
+    L.queue = batch_queue(n, share);
+    if (L.queue) {
+        L.batch_list.assign(2 * items, 0);
+        for (uint32_t item = 0; item < items; ++item) entry(&L.batch_list[2 * static_cast<size_t>(item)], item);
+    } else {
+        std::vector<uint32_t> &deal = n == 1 ? L.deal : L.batch_list;
         const std::vector<uint32_t> lists = deal_items(item_costs(L), workgroup_weights(L.workgroups, cus));
         const uint32_t head = (L.workgroups + 2) & ~1u;
-        L.deal.assign(head + 2 * items, 0);
-        std::copy(lists.begin(), lists.begin() + L.workgroups + 1, L.deal.begin());
-        std::vector<uint32_t> owner(items);
-        for (uint32_t i = 0; i < count; ++i)
-            for (uint32_t item = L.descs[i].item_begin; item < L.descs[i + 1].item_begin; ++item) owner[item] = i;
-        for (uint64_t k = 0; k < items; ++k) {
-            const uint32_t item = lists[L.workgroups + 1 + k];
-            L.deal[head + 2 * k] = owner[item];
-            L.deal[head + 2 * k + 1] = item - L.descs[owner[item]].item_begin;
-        }
+        deal.assign(head + 2 * items, 0);
+        std::copy(lists.begin(), lists.begin() + L.workgroups + 1, deal.begin());
+        for (uint64_t k = 0; k < items; ++k) entry(&deal[head + 2 * k], lists[L.workgroups + 1 + k]);
     }
     L.deal_off = align256(L.table_off + L.table_bytes);
-    L.tail_off = align256(L.deal_off + L.deal.size() * sizeof(uint32_t));
+    L.tail_off = align256(L.deal_off + (L.deal.size() + L.batch_list.size()) * sizeof(uint32_t));
     L.scratch_bytes = L.tail_off + tail;
     L.table.assign(n == 1 ? groups : (groups + 1) / 2, 0);
     for (uint32_t i = 0; i < count; ++i)

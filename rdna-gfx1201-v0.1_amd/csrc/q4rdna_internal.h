@@ -86,6 +86,8 @@ struct PlanDesc {
     uint32_t streams;
     uint32_t per;
     uint32_t pair;  // single vector, no gate, one chunk: an item covers two 64-row blocks (128 rows)
+    uint32_t chunk_groups;  // groups of a K chunk (the last may hold fewer)
+    uint32_t reserved;
 };
 
 // The single-vector sweep's arithmetic: the int8-MFMA formulation, or, in
@@ -151,9 +153,10 @@ uint32_t gemv_multi_stage_groups(uint32_t vectors);
 // items, dealt to its workgroups by the plan: deal holds workgroups + 1
 // offsets (padded to an even count), then one (descriptor index, item within
 // the descriptor) pair of uint32 per item; workgroup b runs entries
-// [deal[b], deal[b + 1]), in increasing item order.  The batched sweep takes items from a queue instead: sched
-// holds its two zeroed counters, owned by the plan (left zero after every
-// launch).
+// [deal[b], deal[b + 1]), in increasing item order.  The batched sweep takes such a deal as
+// its list, or with `queue` claims its items: then list holds the pairs in
+// item order, without offsets, sched is the queue's two zeroed counters,
+// owned by the plan (left zero after every launch), and workgroups <= items.
 hipError_t launch_prep(const float *const *group_x, uint8_t *prep, uint32_t groups, hipStream_t stream);
 // both_streams: some GEMV has per == 1 with a SwiGLU gate (one item streams
 // both weights); plans without such GEMVs run a sweep built without that path.
@@ -163,16 +166,22 @@ hipError_t launch_plan(const PlanDesc *descs, const uint32_t *deal, uint32_t wor
 // plus a fixed charge for its end (reduction, stores, barrier), measured at
 // about the time one workgroup takes to stream eight tiles.
 constexpr uint32_t kItemEndTiles = 8;
+// The same for batched items.
+constexpr uint32_t kBatchItemEndTiles = 16;
 // Batched plans (n = 2..8 activation vectors per GEMV; x [n][cols],
 // y and add [n][rows]): items are 256-row blocks, prep holds
 // kBatchQuadBytesHost per (group, quad of 4 vectors).
 constexpr uint32_t kBatchQuadBytesHost = 1040;
 constexpr uint32_t kBatchBlockRows = 256;
-constexpr uint32_t kBatchChunkGroups = 192;  // K chunk of a batched item (a whole 12288-wide row)
+// Largest K chunk of a batched item (a whole 12288-wide row), and the
+// smallest that layout_plan cuts rows into where a plan has little work
+// (half of it where a workgroup has less than two steps).
+constexpr uint32_t kBatchChunkGroups = 192;
+constexpr uint32_t kMinBatchChunkGroups = 32;
 hipError_t launch_prep_batch(const PlanDesc *descs, const uint32_t *owner, uint32_t groups, uint32_t n,
                              hipStream_t stream);
-hipError_t launch_plan_batch(const PlanDesc *descs, uint32_t items, uint32_t n, uint32_t workgroups, uint32_t *sched,
-                             hipStream_t stream);
+hipError_t launch_plan_batch(const PlanDesc *descs, const uint32_t *list, bool queue, uint32_t items, uint32_t n,
+                             uint32_t workgroups, uint32_t *sched, hipStream_t stream);
 constexpr uint32_t kMaxGroup = 8;  // GEMVs of one group launch (Q4RDNA_MAX_GROUP)
 
 // A VALU group launch (gemv_kernel's arithmetic): up to kMaxGroup GEMVs

@@ -31,6 +31,8 @@
 //    activation digits are stored in the same order.
 //
 // The sweep kernel's lane mapping is described at the kernel below.
+#include <type_traits>
+
 #include "q4rdna_device.h"
 
 namespace q4rdna {
@@ -978,10 +980,9 @@ constexpr int kBatchWaves = 4;  // eight waves per workgroup measured slower
 
 // A wave's stage also receives its partial sums at the item's end (after
 // its last step, so the two uses never overlap): 4*NQ x 256 floats <= 8 KB.
-template <int NQ>
 struct BatchShared {
     uint8_t stage[kBatchWaves][kStageBytes];
-    uint32_t next_item[2];
+    uint3 next_item;  // the next item's number and table entry
     uint32_t last;
 };
 static_assert(8 * kBatchRows * sizeof(float) <= kStageBytes, "partials must fit a wave's stage");
@@ -1021,48 +1022,72 @@ __device__ __forceinline__ void compute_batch(const BatchRegs &r, const i32x4 (&
     }
 }
 
-template <int NQ>
-__device__ __forceinline__ void run_batch_item(BatchShared<NQ> &sh, const PlanDesc &d, uint32_t local, uint32_t nvec,
-                                               int lane, int wave) {
+// Item `local` of GEMV d, decoded.  A SwiGLU GEMV whose rows fit one chunk has
+// one item per block that streams up, then gate, into the same accumulators
+// (no partials).
+struct BatchItem {
+    const uint8_t *w, *gate;  // the item's first stream; the gate of a both-streams item
+    const uint8_t *prep;
+    const float *add;
+    float *y;
+    float *partial;
+    uint32_t *counters;
+    size_t row_tile_bytes;
+    uint32_t rows, tiles, block, part, per, chunks, streams, g_begin, g_end;
+    bool both;
+};
+
+__device__ __forceinline__ BatchItem decode_batch_item(const PlanDesc &d, uint32_t local) {
+    BatchItem c;
     const uint32_t groups = d.cols / kGroup;
-    const uint32_t tiles = d.rows / kTileRows;
-    const uint32_t per = d.per;
-    // A SwiGLU GEMV whose rows fit one chunk has one item per block that
-    // streams up, then gate, into two accumulator sets (no partials).
-    const bool both = d.streams > 1 && per == 1;
-    const uint32_t block = local / per, part = local - block * per;
-    const uint32_t stream = part / d.chunks, chunk = part - stream * d.chunks;
-    const uint32_t g_begin = chunk * kBatchChunkGroups;
-    const uint32_t g_end = min(groups, g_begin + kBatchChunkGroups);
-    const size_t row_tile_bytes = static_cast<size_t>(groups) * kTileBytes;
-    const uint8_t *base = stream != 0 ? d.gate : d.w;
+    c.per = d.per;
+    c.chunks = d.chunks;
+    c.streams = d.streams;
+    c.both = d.streams > 1 && d.per == 1;
+    c.block = local / d.per;
+    c.part = local - c.block * d.per;
+    const uint32_t stream = c.part / d.chunks, chunk = c.part - stream * d.chunks;
+    c.g_begin = chunk * d.chunk_groups;
+    c.g_end = min(groups, c.g_begin + d.chunk_groups);
+    c.w = stream != 0 ? d.gate : d.w;
+    c.gate = d.gate;
+    c.prep = d.prep;
+    c.add = d.add;
+    c.y = d.y;
+    c.partial = d.partial;
+    c.counters = d.counters;
+    c.rows = d.rows;
+    c.tiles = d.rows / kTileRows;
+    c.row_tile_bytes = static_cast<size_t>(groups) * kTileBytes;
+    return c;
+}
+
+// Group g of a block's eight row tiles: those past the last re-read the last
+// (their rows are never written).
+__device__ __forceinline__ void load_batch_step(const uint8_t *w, const BatchItem &c, uint32_t g, int lane, BatchRegs &r) {
+    const uint8_t *at = w + static_cast<size_t>(g) * kTileBytes;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        r.code[i] = __builtin_nontemporal_load(
+            (gptr_i32x4)(at + static_cast<size_t>(min(8 * c.block + i, c.tiles - 1)) * c.row_tile_bytes + 64 + 16 * lane));
+    const uint32_t T = (lane & 15) >> 1, h = lane & 1;
+    const uint8_t *own = at + static_cast<size_t>(min(8 * c.block + T, c.tiles - 1)) * c.row_tile_bytes + 32 * h;
+    r.sc[0] = __builtin_nontemporal_load((gptr_i32x4)own);
+    r.sc[1] = __builtin_nontemporal_load((gptr_i32x4)(own + 16));
+}
+
+// The wave's steps over groups g, g + kBatchWaves, .. of one stream; with
+// have_pre the first one's loads are in `pre`.
+template <int NQ>
+__device__ __forceinline__ void batch_steps(uint8_t *stage, const uint8_t *w, const BatchItem &c, int lane, int wave,
+                                            BatchRegs &pre, bool have_pre, float (&acc)[NQ][16]) {
     const int kslot = lane >> 4, j = lane & 15, T = j >> 1, h = j & 1;
     const uint32_t lds_read = kStageStride * T + 32 * kslot + 16 * h;
-    // The block's eight row tiles; those past the last re-read the last
-    // (their rows are never written).
-    const uint8_t *rt[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) rt[c] = base + static_cast<size_t>(min(8 * block + c, tiles - 1)) * row_tile_bytes;
     const size_t prep_stride = static_cast<size_t>(NQ) * kBatchQuadBytes;
-    float acc[NQ][16];
-#pragma unroll
-    for (int vq = 0; vq < NQ; ++vq)
-#pragma unroll
-        for (int n = 0; n < 16; ++n) acc[vq][n] = 0.0f;
-
-    auto load = [&](uint32_t g, BatchRegs &r) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-            r.code[c] = __builtin_nontemporal_load((gptr_i32x4)(rt[c] + static_cast<size_t>(g) * kTileBytes + 64 + 16 * lane));
-        const uint8_t *own = rt[T] + static_cast<size_t>(g) * kTileBytes + 32 * h;
-        r.sc[0] = __builtin_nontemporal_load((gptr_i32x4)own);
-        r.sc[1] = __builtin_nontemporal_load((gptr_i32x4)(own + 16));
-        __builtin_amdgcn_sched_barrier(0);
-    };
     auto step = [&](uint32_t g, BatchRegs &r) {
         i32x4 a[NQ];
         float f[NQ];
-        const uint8_t *pg = d.prep + static_cast<size_t>(g) * prep_stride;
+        const uint8_t *pg = c.prep + static_cast<size_t>(g) * prep_stride;
 #pragma unroll
         for (int vq = 0; vq < NQ; ++vq) {
             a[vq] = *(gptr_i32x4)(pg + vq * kBatchQuadBytes + 256 * kslot + 16 * j);
@@ -1071,160 +1096,205 @@ __device__ __forceinline__ void run_batch_item(BatchShared<NQ> &sh, const PlanDe
         // Restaged through registers: loading straight into LDS, as the
         // single-vector sweep does, measured neutral to 0.6 % slower here.
 #pragma unroll
-        for (int c = 0; c < 8; ++c) *reinterpret_cast<i32x4 *>(sh.stage[wave] + kStageStride * c + 16 * lane) = r.code[c];
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<i32x4 *>(stage + kStageStride * i + 16 * lane) = r.code[i];
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int c = 0; c < 8; ++c) r.code[c] = *reinterpret_cast<const i32x4 *>(sh.stage[wave] + lds_read + 128 * c);
+        for (int i = 0; i < 8; ++i) r.code[i] = *reinterpret_cast<const i32x4 *>(stage + lds_read + 128 * i);
         compute_batch<NQ>(r, a, f, acc);
     };
     // One step in flight per wave: each step's loads follow the previous
     // step's arithmetic (two steps in flight measured slower, as in the
-    // single-vector sweep).  Loading the next item's first step across this
-    // item's end, after the barrier that follows the last step (the next
-    // item is claimed one ahead), measured 0.6-1.3 % slower at N = 2, 4, 8.
+    // single-vector sweep).
+    uint32_t g = c.g_begin + wave;
+    if (have_pre) {
+        step(g, pre);
+        g += kBatchWaves;
+    }
+    for (; g < c.g_end; g += kBatchWaves) {
+        BatchRegs r;
+        load_batch_step(w, c, g, lane, r);
+        __builtin_amdgcn_sched_barrier(0);
+        step(g, r);
+    }
+}
+
+// The end of an item, after the waves' partials (and the workgroup barrier):
+// thread t finishes row t of the block (blockDim.x == kBatchRows).  u holds
+// the up sums of a both-streams item.
+template <int NQ, class Total>
+__device__ __forceinline__ void finish_batch_item(uint32_t &last, const BatchItem &c, uint32_t nvec, Total total,
+                                                  const float (&u)[4 * NQ]) {
+    const uint32_t r = threadIdx.x, row = c.block * kBatchRows + r;
+    const size_t M = c.rows;
+    const bool mine = row < c.rows;
+    if (c.both) {
+        // y = (up + add) * silu(gate), the up sums from registers.
+        if (mine) {
+#pragma unroll
+            for (int vec = 0; vec < 4 * NQ; ++vec) {
+                if (static_cast<uint32_t>(vec) >= nvec) break;
+                float v = u[vec];
+                if (c.add != nullptr) v += ((gptr_cf32)c.add)[vec * M + row];
+                __builtin_nontemporal_store(v * silu(total(vec, r)), (gptr_f32)c.y + vec * M + row);
+            }
+        }
+        return;
+    }
+    if (c.per == 1) {
+        if (mine) {
+            for (uint32_t vec = 0; vec < nvec; ++vec) {
+                float v = total(vec, r);
+                if (c.add != nullptr) v += ((gptr_cf32)c.add)[vec * M + row];
+                __builtin_nontemporal_store(v, (gptr_f32)c.y + vec * M + row);
+            }
+        }
+        return;
+    }
+    if (mine) {
+        for (uint32_t vec = 0; vec < nvec; ++vec)
+            store_agent(&c.partial[(static_cast<size_t>(c.part) * nvec + vec) * M + row], total(vec, r));
+    }
+    wait_stores();
+    __syncthreads();
+    if (threadIdx.x == 0) last = (add_agent(&c.counters[c.block], 1u) == c.per - 1) ? 1u : 0u;
+    __syncthreads();
+    if (last == 0u) return;
+    if (mine) {
+        for (uint32_t vec = 0; vec < nvec; ++vec) {
+            float v = load_agent(&c.partial[static_cast<size_t>(vec) * M + row]);
+            for (uint32_t k = 1; k < c.chunks; ++k) v += load_agent(&c.partial[(static_cast<size_t>(k) * nvec + vec) * M + row]);
+            if (c.add != nullptr) v += ((gptr_cf32)c.add)[vec * M + row];
+            if (c.streams > 1) {
+                float g = load_agent(&c.partial[(static_cast<size_t>(c.chunks) * nvec + vec) * M + row]);
+                for (uint32_t k = 1; k < c.chunks; ++k)
+                    g += load_agent(&c.partial[(static_cast<size_t>(c.chunks + k) * nvec + vec) * M + row]);
+                v *= silu(g);
+            }
+            __builtin_nontemporal_store(v, (gptr_f32)c.y + vec * M + row);
+        }
+    }
+    if (threadIdx.x == 0) store_agent(&c.counters[c.block], 0u);
+}
+
+// QUEUE: workgroup b runs item b, then items claimed from a queue; list[item]
+// is an item's descriptor and its index within it (walking the GEMVs' item
+// ranges instead cost a dependent load per GEMV passed).  Thread 0 claims two
+// items ahead and reads the next one's entry while an item's steps run, so
+// that neither round trip is waited for.  Otherwise list is a deal, as
+// plan_kernel's, and every wave loads the next item's first step across an
+// item's end.  batch_queue (q4rdna_host.cpp) says which a plan takes.
+template <int NQ, bool QUEUE>
+__global__ __launch_bounds__(64 * kBatchWaves, 2) void plan_batch_kernel(const PlanDesc *__restrict__ descs,
+                                                                         const uint32_t *__restrict__ list, uint32_t items,
+                                                                         uint32_t nvec, uint32_t *__restrict__ sched) {
+    __shared__ BatchShared sh;
+    const int lane = threadIdx.x & 63, wave = wave_id();
+#if defined(Q4RDNA_SWEEP_CLOCKS)
+    const uint64_t clock_start = __builtin_amdgcn_s_memrealtime();
+#endif
+    const uint2 *entry = reinterpret_cast<const uint2 *>(QUEUE ? list : list + ((gridDim.x + 2) & ~1u));
+    // The item's entry, and the end of the entries that are the workgroup's
+    // (a queued plan launches at most `items` workgroups).
+    uint32_t k = QUEUE ? blockIdx.x : list[blockIdx.x];
+    const uint32_t end = QUEUE ? items : list[blockIdx.x + 1];
+    if (k >= end) return;
+    auto locate = [&](uint2 e) { return decode_batch_item(descs[e.x], e.y); };
+    BatchItem cur = locate(entry[k]);
+    auto claim = [&]() { return gridDim.x + add_agent(&sched[0], 1u); };
+    uint32_t claimed = 0;  // thread 0 of a queued sweep: the next item
+    if (QUEUE && threadIdx.x == 0) claimed = claim();
+    BatchRegs pre;
+    bool have_pre = false;
+    const int kslot = lane >> 4, T = (lane & 15) >> 1, h = lane & 1;
     // Lane (kslot, j) holds vector 4*vq + kslot, rows 32T + 16h + n; the
     // wave's partials go to red[vector][row] in its own stage.
     float *red = reinterpret_cast<float *>(sh.stage[wave]);
-    auto publish = [&]() {
+    auto publish = [&](const float (&acc)[NQ][16]) {
 #pragma unroll
         for (int vq = 0; vq < NQ; ++vq) {
-            const uint32_t vec = 4 * vq + kslot;
-            if (vec < nvec) {
+            if (4 * vq + kslot < static_cast<int>(nvec)) {
                 float *dst = red + (4 * vq + kslot) * kBatchRows + 32 * T + 16 * h;
 #pragma unroll
                 for (int n = 0; n < 16; ++n) dst[n] = acc[vq][n];
             }
         }
     };
-    // Threads split the block's rows; each sums its rows' partials over the
-    // waves in wave order.
+    // A row's partials over the waves, in wave order.
     auto total = [&](uint32_t vec, uint32_t r) {
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < kBatchWaves; ++w) v += reinterpret_cast<const float *>(sh.stage[w])[vec * kBatchRows + r];
         return v;
     };
-
-    for (uint32_t g = g_begin + wave; g < g_end; g += kBatchWaves) {
-        BatchRegs r;
-        load(g, r);
-        step(g, r);
-    }
-    // Both streams: the up sums go to registers, one row per thread
-    // (blockDim.x == kBatchRows), and the accumulators start over on the gate.
-    constexpr int V = 4 * NQ;
-    float u[V];
-    if (both) {
-        publish();
-        __syncthreads();
-#pragma unroll
-        for (int vec = 0; vec < V; ++vec) u[vec] = static_cast<uint32_t>(vec) < nvec ? total(vec, threadIdx.x) : 0.0f;
-        __syncthreads();
-#pragma unroll
-        for (int vq = 0; vq < NQ; ++vq)
-#pragma unroll
-            for (int n = 0; n < 16; ++n) acc[vq][n] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-            rt[c] = d.gate + static_cast<size_t>(min(8 * block + c, tiles - 1)) * row_tile_bytes;
-        for (uint32_t g = g_begin + wave; g < g_end; g += kBatchWaves) {
-            BatchRegs r;
-            load(g, r);
-            step(g, r);
+    for (;;) {
+        uint32_t claimed2 = 0;
+        uint2 e = make_uint2(0, 0);
+        if (QUEUE && threadIdx.x == 0) {
+            e = entry[min(claimed, items - 1)];
+            claimed2 = claim();
         }
-    }
-    publish();
-    __syncthreads();
-    const size_t M = d.rows;
-    if (both) {
-        // y = (up + add) * silu(gate), the up sums from registers.
-        const uint32_t r = threadIdx.x, row = block * kBatchRows + r;
-        if (row < d.rows) {
+        if (!QUEUE && k + 1 < end) e = entry[k + 1];
+        float acc[NQ][16], u[4 * NQ];
+        auto clear = [&]() {
 #pragma unroll
-            for (int vec = 0; vec < V; ++vec) {
-                if (static_cast<uint32_t>(vec) >= nvec) break;
-                float v = u[vec];
-                if (d.add != nullptr) v += ((gptr_cf32)d.add)[vec * M + row];
-                __builtin_nontemporal_store(v * silu(total(vec, r)), (gptr_f32)d.y + vec * M + row);
+            for (int vq = 0; vq < NQ; ++vq)
+#pragma unroll
+                for (int n = 0; n < 16; ++n) acc[vq][n] = 0.0f;
+        };
+        clear();
+        batch_steps<NQ>(sh.stage[wave], cur.w, cur, lane, wave, pre, have_pre, acc);
+        // Both streams: the up sums go to registers, one row per thread, and
+        // the accumulators start over on the gate.
+        if (cur.both) {
+            publish(acc);
+            __syncthreads();
+#pragma unroll
+            for (int vec = 0; vec < 4 * NQ; ++vec) u[vec] = static_cast<uint32_t>(vec) < nvec ? total(vec, threadIdx.x) : 0.0f;
+            __syncthreads();
+            clear();
+            batch_steps<NQ>(sh.stage[wave], cur.gate, cur, lane, wave, pre, false, acc);
+        }
+        publish(acc);
+        BatchItem next;
+        have_pre = false;
+        if constexpr (QUEUE) {
+            if (threadIdx.x == 0) {
+                sh.next_item = make_uint3(claimed, e.x, e.y);
+                claimed = claimed2;
+            }
+        } else if (++k < end) {
+            next = locate(e);
+            if (next.g_begin + wave < next.g_end) {
+                load_batch_step(next.w, next, next.g_begin + wave, lane, pre);
+                have_pre = true;
             }
         }
-        return;
-    }
-    if (per == 1) {
-        for (uint32_t r = threadIdx.x; r < kBatchRows; r += blockDim.x) {
-            const uint32_t row = block * kBatchRows + r;
-            if (row >= d.rows) break;
-            for (uint32_t vec = 0; vec < nvec; ++vec) {
-                float v = total(vec, r);
-                if (d.add != nullptr) v += ((gptr_cf32)d.add)[vec * M + row];
-                __builtin_nontemporal_store(v, (gptr_f32)d.y + vec * M + row);
-            }
-        }
-        return;
-    }
-    for (uint32_t r = threadIdx.x; r < kBatchRows; r += blockDim.x) {
-        const uint32_t row = block * kBatchRows + r;
-        if (row >= d.rows) break;
-        for (uint32_t vec = 0; vec < nvec; ++vec)
-            store_agent(&d.partial[(static_cast<size_t>(part) * nvec + vec) * M + row], total(vec, r));
-    }
-    wait_stores();
-    __syncthreads();
-    if (threadIdx.x == 0) sh.last = (add_agent(&d.counters[block], 1u) == per - 1) ? 1u : 0u;
-    __syncthreads();
-    if (sh.last == 0u) return;
-    for (uint32_t r = threadIdx.x; r < kBatchRows; r += blockDim.x) {
-        const uint32_t row = block * kBatchRows + r;
-        if (row >= d.rows) break;
-        for (uint32_t vec = 0; vec < nvec; ++vec) {
-            float u = load_agent(&d.partial[static_cast<size_t>(vec) * M + row]);
-            for (uint32_t k = 1; k < d.chunks; ++k) u += load_agent(&d.partial[(static_cast<size_t>(k) * nvec + vec) * M + row]);
-            if (d.add != nullptr) u += ((gptr_cf32)d.add)[vec * M + row];
-            if (d.streams > 1) {
-                float g = load_agent(&d.partial[(static_cast<size_t>(d.chunks) * nvec + vec) * M + row]);
-                for (uint32_t k = 1; k < d.chunks; ++k)
-                    g += load_agent(&d.partial[(static_cast<size_t>(d.chunks + k) * nvec + vec) * M + row]);
-                u *= silu(g);
-            }
-            __builtin_nontemporal_store(u, (gptr_f32)d.y + vec * M + row);
-        }
-    }
-    if (threadIdx.x == 0) store_agent(&d.counters[block], 0u);
-}
-
-template <int NQ>
-__global__ __launch_bounds__(64 * kBatchWaves) void plan_batch_kernel(const PlanDesc *__restrict__ descs, uint32_t items,
-                                                         uint32_t nvec, uint32_t *__restrict__ sched) {
-    __shared__ BatchShared<NQ> sh;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#if defined(Q4RDNA_SWEEP_CLOCKS)
-    const uint64_t clock_start = __builtin_amdgcn_s_memrealtime();
-#endif
-    if (threadIdx.x == 0) sh.next_item[0] = add_agent(&sched[0], 1u);
-    __syncthreads();
-    uint32_t item = sh.next_item[0];
-    uint32_t d = 0;
-    int slot = 0;
-    while (item < items) {
-        if (threadIdx.x == 0) sh.next_item[slot ^ 1] = add_agent(&sched[0], 1u);
-        while (item >= descs[d + 1].item_begin) ++d;
-        run_batch_item<NQ>(sh, descs[d], item - descs[d].item_begin, nvec, lane, wave);
         __syncthreads();
-        slot ^= 1;
-        item = sh.next_item[slot];
+        if constexpr (QUEUE) k = __builtin_amdgcn_readfirstlane(sh.next_item.x);
+        if (QUEUE && k < end)
+            next = locate(make_uint2(__builtin_amdgcn_readfirstlane(sh.next_item.y),
+                                     __builtin_amdgcn_readfirstlane(sh.next_item.z)));
+        finish_batch_item<NQ>(sh.last, cur, nvec, total, u);
+        if (k >= end) break;
+        __syncthreads();  // the partials and the next item are read
+        cur = next;
+    }
+    // The last workgroup to end, with every claim made, empties the queue.
+    if (QUEUE && threadIdx.x == 0) {
+        wait_stores();
+        if (add_agent(&sched[1], 1u) == gridDim.x - 1) {
+            store_agent(&sched[0], 0u);
+            store_agent(&sched[1], 0u);
+        }
     }
 #if defined(Q4RDNA_SWEEP_CLOCKS)
-    // After the last item (the loop ends at a barrier that follows it).
+    __syncthreads();
     if (threadIdx.x == 0 && blockIdx.x < kMaxSweepClocks) {
         const uint64_t clock_end = __builtin_amdgcn_s_memrealtime();
         g_sweep_clocks[2 * blockIdx.x] = clock_start;
         g_sweep_clocks[2 * blockIdx.x + 1] = clock_end;
     }
 #endif
-    if (threadIdx.x == 0 && add_agent(&sched[1], 1u) == gridDim.x - 1) {
-        store_agent(&sched[0], 0u);
-        store_agent(&sched[1], 0u);
-    }
 }
 
 }  // namespace
@@ -1279,13 +1349,22 @@ hipError_t launch_prep_batch(const PlanDesc *descs, const uint32_t *owner, uint3
     return hipGetLastError();
 }
 
-hipError_t launch_plan_batch(const PlanDesc *descs, uint32_t items, uint32_t n, uint32_t workgroups, uint32_t *sched,
-                             hipStream_t stream) {
-    const dim3 block(64 * kBatchWaves);
-    if (n <= 4)
-        hipLaunchKernelGGL(plan_batch_kernel<1>, dim3(workgroups), block, 0, stream, descs, items, n, sched);
+hipError_t launch_plan_batch(const PlanDesc *descs, const uint32_t *list, bool queue, uint32_t items, uint32_t n,
+                             uint32_t workgroups, uint32_t *sched, hipStream_t stream) {
+    const dim3 grid(workgroups), block(64 * kBatchWaves);
+    auto go = [&](auto nq, auto q) {
+        hipLaunchKernelGGL((plan_batch_kernel<decltype(nq)::value, decltype(q)::value>), grid, block, 0, stream, descs, list,
+                           items, n, sched);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if (n > 4 && queue) return hipErrorInvalidValue;  // batch_queue takes it for one quad only
+    if (n > 4)
+        go(Two{}, std::false_type{});
+    else if (queue)
+        go(One{}, std::true_type{});
     else
-        hipLaunchKernelGGL(plan_batch_kernel<2>, dim3(workgroups), block, 0, stream, descs, items, n, sched);
+        go(One{}, std::false_type{});
     return hipGetLastError();
 }
 

@@ -306,12 +306,13 @@ struct q4rdna_plan {
     uint8_t *scratch = nullptr;         // activation digits, split-K partials and counters
     uint32_t *sched = nullptr;          // batched sweeps' [next item, finished workgroups], zero between launches
     uint8_t *table = nullptr;           // prep launch's group table (in scratch)
-    uint32_t *deal = nullptr;           // single-vector sweeps' item deal (in scratch)
+    uint32_t *deal = nullptr;           // the sweep's item deal or queue list (in scratch)
     uint32_t count = 0;
     uint32_t items = 0;
     uint32_t groups = 0;
     uint32_t workgroups = 0;
     uint32_t batch = 1;  // activation vectors per GEMV
+    bool queue = false;         // a batched sweep that claims its items
     bool both_streams = false;  // some SwiGLU GEMV runs both weight streams in one item
 };
 
@@ -830,6 +831,7 @@ int q4rdna_plan_create_batch(const q4rdna_gemv_desc *descs, uint32_t count, uint
     plan->device = device;
     plan->batch = n;
     plan->both_streams = L.both_streams;
+    plan->queue = L.queue;
     plan->count = count;
     for (uint32_t i = 0; i < count; ++i) {
         plan->weights.push_back(descs[i].weight.tiles);
@@ -862,8 +864,9 @@ int q4rdna_plan_create_batch(const q4rdna_gemv_desc *descs, uint32_t count, uint
     e = hipMemcpy(plan->descs, L.descs.data(), L.descs.size() * sizeof(q4rdna::PlanDesc), hipMemcpyHostToDevice);
     if (e == hipSuccess && L.scratch_bytes > 0) e = hipMemset(plan->scratch, 0, L.scratch_bytes);
     if (e == hipSuccess && L.groups > 0) e = hipMemcpy(plan->table, L.table.data(), L.table_bytes, hipMemcpyHostToDevice);
-    if (e == hipSuccess && !L.deal.empty())
-        e = hipMemcpy(plan->deal, L.deal.data(), L.deal.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
+    const std::vector<uint32_t> &entries = n == 1 ? L.deal : L.batch_list;
+    if (e == hipSuccess && !entries.empty())
+        e = hipMemcpy(plan->deal, entries.data(), entries.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(plan->sched, 0, 2 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
@@ -905,8 +908,8 @@ int q4rdna_plan_sweep(q4rdna_plan *plan, void *stream) {
     hipError_t e = plan->batch == 1
                        ? q4rdna::launch_plan(plan->descs, plan->deal, plan->workgroups, plan->both_streams,
                                              static_cast<hipStream_t>(stream))
-                       : q4rdna::launch_plan_batch(plan->descs, plan->items, plan->batch, plan->workgroups,
-                                                   plan->sched, static_cast<hipStream_t>(stream));
+                       : q4rdna::launch_plan_batch(plan->descs, plan->deal, plan->queue, plan->items, plan->batch,
+                                                   plan->workgroups, plan->sched, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "plan sweep launch");
     count_launch(plan->weights.data(), plan->weights.size());
     return Q4RDNA_OK;
