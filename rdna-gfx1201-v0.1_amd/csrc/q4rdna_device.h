@@ -221,6 +221,43 @@ __device__ __forceinline__ void apply_codes(const TileCodes &w, uint32_t s01, ui
     acc[3] = fmaf(half_bits_to_float(s23 >> 16), p3, acc[3]);
 }
 
+// fma(half h, x, p) in one instruction, H = 0 the low half of h, 1 the high.
+// Written out because the compiler converts a code that several vectors use
+// once and keeps it: a conversion per code, and twice the registers.
+template <int H>
+__device__ __forceinline__ float fma_mix(f16x2 h, float x, float p) {
+    float r;
+    if constexpr (H == 0)
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x), "v"(p));
+    else
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x), "v"(p));
+    return r;
+}
+
+// apply_codes, step by step, with fma_mix.
+__device__ __forceinline__ void apply_codes_mix(const TileCodes &w, uint32_t s01, uint32_t s23, const float4 xl,
+                                                const float4 xh, const float c, float (&acc)[4]) {
+    const float xlv[4] = {xl.x, xl.y, xl.z, xl.w};
+    const float xhv[4] = {xh.x, xh.y, xh.z, xh.w};
+    float p0 = c, p1 = c, p2 = c, p3 = c;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        p0 = fma_mix<0>(w.l02[j], xlv[j], p0);
+        p1 = fma_mix<0>(w.l13[j], xlv[j], p1);
+        p2 = fma_mix<1>(w.l02[j], xlv[j], p2);
+        p3 = fma_mix<1>(w.l13[j], xlv[j], p3);
+        p0 = fma_mix<0>(w.h02[j], xhv[j], p0);
+        p1 = fma_mix<0>(w.h13[j], xhv[j], p1);
+        p2 = fma_mix<1>(w.h02[j], xhv[j], p2);
+        p3 = fma_mix<1>(w.h13[j], xhv[j], p3);
+    }
+    const f16x2 a = __builtin_bit_cast(f16x2, s01), b = __builtin_bit_cast(f16x2, s23);
+    acc[0] = fma_mix<0>(a, p0, acc[0]);
+    acc[1] = fma_mix<1>(a, p1, acc[1]);
+    acc[2] = fma_mix<0>(b, p2, acc[2]);
+    acc[3] = fma_mix<1>(b, p3, acc[3]);
+}
+
 // Activation factors for apply_codes: x * 2^24 at even k, x * 2^20 at odd
 // k (the 1/16 of the high nibbles folded in); every product is then exactly
 // u * x.  The staged values are finite for |x| < 2^104.

@@ -435,7 +435,17 @@ struct MvShared {
     float red[2][NV][kMvWaves][32];
 };
 
-template <bool GATE, bool ADD, int NV, int T>
+// MIX: how a code that several vectors share enters their sums, as fp16 in
+// each fma (fma_mix) or converted once.  The bits are the same.  The fp16 form
+// takes 68 registers instead of 84 (NV = 8) and at most 124 instead of 156
+// with a gate, so one more workgroup fits a CU, and no conversions; the other
+// is faster where the workgroups fit anyway.  us, converted / fp16:
+//   12288x4096 with a gate   n = 2 22.9 / 17.8, n = 4 30.4 / 23.0, n = 8 49.1 / 38.0
+//   2048x28672               n = 2 13.9 / 12.4, n = 4 17.0 / 17.0, n = 5 23.5 / 21.3, n = 7 26.8 / 27.2
+//   4096x4096                n = 2 5.93 / 5.74, n = 4 7.73 / 7.91, n = 5 8.44 / 8.73, n = 8 10.0 / 10.7
+// So fp16 with a gate, for two vectors, and for five or six where the launch
+// has more than two workgroups per CU (launch_multi_nv).
+template <bool GATE, bool ADD, int NV, int T, bool MIX>
 __global__ __launch_bounds__(64 * kMvWaves) void gemv_multi_kernel(GemvArgs args) {
     constexpr int W = kMvWaves;
     constexpr int SG = mv_stage_groups<NV>();
@@ -521,8 +531,13 @@ __global__ __launch_bounds__(64 * kMvWaves) void gemv_multi_kernel(GemvArgs args
                     const float4 xl = sh.v[v][gg][a];
                     const float4 xh = sh.v[v][gg][8 + a];
                     const float c = sh.c[v][gg][a];
-                    apply_codes(w, t[i].s01, t[i].s23, xl, xh, c, acc[v]);
-                    if constexpr (GATE) apply_codes(gw, u[i].s01, u[i].s23, xl, xh, c, gacc[v]);
+                    if constexpr (MIX) {
+                        apply_codes_mix(w, t[i].s01, t[i].s23, xl, xh, c, acc[v]);
+                        if constexpr (GATE) apply_codes_mix(gw, u[i].s01, u[i].s23, xl, xh, c, gacc[v]);
+                    } else {
+                        static_assert(!GATE, "SwiGLU launches take the fp16 form");
+                        apply_codes(w, t[i].s01, t[i].s23, xl, xh, c, acc[v]);
+                    }
                 }
             }
         }
@@ -1044,20 +1059,31 @@ hipError_t launch_gemv_t(const GemvArgs &args, hipStream_t stream) {
                                            : launch_gemv_w<GATE, ADD, kWaves>(args, stream);
 }
 
-template <bool GATE, bool ADD, int NV>
-hipError_t launch_multi_nv(const GemvArgs &args, hipStream_t stream) {
+template <bool GATE, bool ADD, int NV, bool MIX>
+hipError_t launch_multi_mix(const GemvArgs &args, hipStream_t stream) {
     constexpr int W = kMvWaves;
     const uint32_t blocks = (args.rows / kTileRows) * args.split;
     const uint32_t groups = args.cols / kGroup;
     const uint32_t per_wave = ((groups + args.split - 1) / args.split + W - 1) / W;
     const dim3 grid(blocks), block(64 * W);
     if (per_wave <= 1)
-        hipLaunchKernelGGL((gemv_multi_kernel<GATE, ADD, NV, 1>), grid, block, 0, stream, args);
+        hipLaunchKernelGGL((gemv_multi_kernel<GATE, ADD, NV, 1, MIX>), grid, block, 0, stream, args);
     else if (per_wave <= 2 || NV >= 8)
-        hipLaunchKernelGGL((gemv_multi_kernel<GATE, ADD, NV, 2>), grid, block, 0, stream, args);
+        hipLaunchKernelGGL((gemv_multi_kernel<GATE, ADD, NV, 2, MIX>), grid, block, 0, stream, args);
     else
-        hipLaunchKernelGGL((gemv_multi_kernel<GATE, ADD, NV, (NV >= 8 ? 2 : 4)>), grid, block, 0, stream, args);
+        hipLaunchKernelGGL((gemv_multi_kernel<GATE, ADD, NV, (NV >= 8 ? 2 : 4), MIX>), grid, block, 0, stream, args);
     return hipGetLastError();
+}
+
+template <bool GATE, bool ADD, int NV>
+hipError_t launch_multi_nv(const GemvArgs &args, hipStream_t stream) {
+    if constexpr (GATE || NV == 2)
+        return launch_multi_mix<GATE, ADD, NV, true>(args, stream);
+    else if constexpr (NV == 4)
+        return launch_multi_mix<GATE, ADD, NV, false>(args, stream);
+    else
+        return args.crowded && args.vectors <= 6 ? launch_multi_mix<GATE, ADD, NV, true>(args, stream)
+                                                : launch_multi_mix<GATE, ADD, NV, false>(args, stream);
 }
 
 template <bool GATE, bool ADD>
