@@ -56,7 +56,7 @@ struct GemvArgs {
     uint32_t vectors;      // launch_gemv_multi: activation vectors (x [vectors][cols], y/add [vectors][rows])
     uint32_t split_magic;  // split_magic(split)
     uint32_t clock_slot;   // the clock build's record slot for this launch
-    uint32_t crowded;      // launch_gemv_multi: more than two workgroups per CU
+    uint32_t per_cu;       // launch_gemv_multi: workgroups per CU, rounded up
 };
 
 // Device-side descriptor of one GEMV in a multi-tensor plan.  Work items are

@@ -442,9 +442,11 @@ struct MvShared {
 // is faster where the workgroups fit anyway.  us, converted / fp16:
 //   12288x4096 with a gate   n = 2 22.9 / 17.8, n = 4 30.4 / 23.0, n = 8 49.1 / 38.0
 //   2048x28672               n = 2 13.9 / 12.4, n = 4 17.0 / 17.0, n = 5 23.5 / 21.3, n = 7 26.8 / 27.2
+//   1024x1024 with a gate    n = 4 6.16 / 6.32, n = 8 8.70 / 9.40
 //   4096x4096                n = 2 5.93 / 5.74, n = 4 7.73 / 7.91, n = 5 8.44 / 8.73, n = 8 10.0 / 10.7
-// So fp16 with a gate, for two vectors, and for five or six where the launch
-// has more than two workgroups per CU (launch_multi_nv).
+// So fp16 for two vectors, with a gate where the launch has more than one
+// workgroup per CU, and for five or six vectors where it has more than two
+// (launch_multi_nv).
 template <bool GATE, bool ADD, int NV, int T, bool MIX>
 __global__ __launch_bounds__(64 * kMvWaves) void gemv_multi_kernel(GemvArgs args) {
     constexpr int W = kMvWaves;
@@ -535,8 +537,8 @@ __global__ __launch_bounds__(64 * kMvWaves) void gemv_multi_kernel(GemvArgs args
                         apply_codes_mix(w, t[i].s01, t[i].s23, xl, xh, c, acc[v]);
                         if constexpr (GATE) apply_codes_mix(gw, u[i].s01, u[i].s23, xl, xh, c, gacc[v]);
                     } else {
-                        static_assert(!GATE, "SwiGLU launches take the fp16 form");
                         apply_codes(w, t[i].s01, t[i].s23, xl, xh, c, acc[v]);
+                        if constexpr (GATE) apply_codes(gw, u[i].s01, u[i].s23, xl, xh, c, gacc[v]);
                     }
                 }
             }
@@ -1077,13 +1079,15 @@ hipError_t launch_multi_mix(const GemvArgs &args, hipStream_t stream) {
 
 template <bool GATE, bool ADD, int NV>
 hipError_t launch_multi_nv(const GemvArgs &args, hipStream_t stream) {
-    if constexpr (GATE || NV == 2)
+    if constexpr (NV == 2) {
         return launch_multi_mix<GATE, ADD, NV, true>(args, stream);
-    else if constexpr (NV == 4)
+    } else if constexpr (!GATE && NV == 4) {
         return launch_multi_mix<GATE, ADD, NV, false>(args, stream);
-    else
-        return args.crowded && args.vectors <= 6 ? launch_multi_mix<GATE, ADD, NV, true>(args, stream)
-                                                : launch_multi_mix<GATE, ADD, NV, false>(args, stream);
+    } else {
+        const bool mix = GATE ? args.per_cu > 1 : args.per_cu > 2 && args.vectors <= 6;
+        return mix ? launch_multi_mix<GATE, ADD, NV, true>(args, stream)
+                   : launch_multi_mix<GATE, ADD, NV, false>(args, stream);
+    }
 }
 
 template <bool GATE, bool ADD>

@@ -799,7 +799,8 @@ int q4rdna_mul_mat_batch(const q4rdna_weight *w, const q4rdna_weight *gate, cons
     args.split = split;
     args.split_magic = q4rdna::split_magic(split);
     args.vectors = n;
-    args.crowded = static_cast<uint64_t>(w->rows / kTileRows) * split > 2ull * cu_count(w->device);
+    const uint64_t cus = cu_count(w->device);
+    args.per_cu = static_cast<uint32_t>((static_cast<uint64_t>(w->rows / kTileRows) * split + cus - 1) / cus);
     if (split > 1) {
         Workspace *ws = nullptr;
         const size_t sc = static_cast<size_t>(q4rdna::host::exchange_nodes(split)) * n * w->rows * (gate ? 2 : 1);

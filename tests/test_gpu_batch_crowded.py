@@ -1,6 +1,6 @@
-"""q4rdna_mul_mat_batch on either side of the line where its codes enter the
-sums in another form (more than two workgroups per CU, five or six vectors):
-every vector equals q4rdna_mul_mat_ex of it at the same split bit for bit."""
+"""q4rdna_mul_mat_batch on either side of the lines where its codes enter the
+sums in another form (more than one workgroup per CU with a gate, more than two
+without and five or six vectors): every vector equals q4rdna_mul_mat_ex of it at the same split bit for bit."""
 import pytest
 import torch
 
@@ -11,8 +11,8 @@ from test_gpu_parity import dev_f32, dev_u8, random_tiles
 pytestmark = pytest.mark.gpu
 
 
-# 512 workgroups are two per CU; single launches run eight waves up to 1024.
-@pytest.mark.parametrize("rows", [32 * 256, 32 * 257, 32 * 512])
+# 256 workgroups are one per CU; single launches run eight waves up to 1024.
+@pytest.mark.parametrize("rows", [32 * 128, 32 * 129, 32 * 256, 32 * 257, 32 * 512])
 @pytest.mark.parametrize("n", [2, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("kind", ["plain", "add", "glu"])
 def test_batch_equals_single(cuda, rows, n, kind):
