@@ -181,8 +181,9 @@ int q4rdna_mul_mat_ex(const q4rdna_weight *w, const q4rdna_weight *gate, const f
  * floats back to back, y (and add) n rows of `rows` floats, as ggml's src1
  * and dst with ne[1] = n, contiguous.  gate (may be NULL) makes it the
  * SwiGLU site.  options->split_k as in q4rdna_mul_mat_ex (0 = the shape
- * policy); for n >= 2 it is raised until every K chunk holds at most 32
- * groups (16 for n > 4).  Each tile is read once for all n vectors; each
+ * policy, for n >= 2 with its own choice for tall and uneven shapes); for
+ * n >= 2 it is raised until every K chunk holds at most 32 groups (16 for
+ * n > 4).  Each tile is read once for all n vectors; each
  * vector's result is bit-identical to q4rdna_mul_mat_ex of that vector with
  * that split where that call runs eight-wave workgroups. */
 int q4rdna_mul_mat_batch(const q4rdna_weight *w, const q4rdna_weight *gate, const float *x, uint32_t n,
@@ -218,7 +219,8 @@ typedef struct q4rdna_group_desc {
 int q4rdna_mul_mat_group(const q4rdna_group_desc *descs, uint32_t count, const float *x, int64_t x_ne0,
                          const q4rdna_launch_options *options, void *stream);
 
-/* Split-K factor the shape policy picks for rows x columns on `device`. */
+/* Split-K factor the shape policy picks for rows x columns on `device`,
+ * without a SwiGLU gate (single launches with one may take more chunks). */
 uint32_t q4rdna_policy_split_k(uint32_t rows, uint32_t columns, int device);
 
 /* q4rdna_mul_mat_ex that allocates nothing.  No counterpart in the

@@ -71,20 +71,38 @@ bool valid_shape(uint32_t rows, uint32_t cols) {
     return rows > 0 && cols > 0 && rows % kTileRows == 0 && cols % kGroup == 0;
 }
 
-uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus) {
+uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus, uint32_t streams, uint32_t vectors) {
     // About 32 groups per workgroup (eight waves of four tiles, all in flight
     // at once) and at most 8 chunks; more chunks only when the row tiles are
-    // so few that under a quarter of the CUs would get a workgroup, fewer
-    // when there would be more than six workgroups per CU.  Measured on
-    // MI355X (split sweep, with and without a SwiGLU gate): 4096x4096 best at
-    // 2, 1024x4096 at 2-4, 12288x4096 at 2, 4096x12288 at 6, 2048x28672 at
+    // so few that under a quarter of the CUs would get a workgroup.  Measured
+    // on MI355X (split sweep, with and without a SwiGLU gate): 4096x4096 best
+    // at 2, 1024x4096 at 2-4, 12288x4096 at 2, 4096x12288 at 6, 2048x28672 at
     // 7-8, 151936x4096 at 1-2.
+    //
+    // A wave holds 1, 2, 4 or 8 tiles, so 16 groups per workgroup are taken
+    // where they fill the waves better than 32 (41 groups: three chunks of 14
+    // instead of two of 21), and with a gate, whose chunks are twice the
+    // bytes, once that makes more than six workgroups per CU (12288x4096 with
+    // a gate, six, measures 12.5 us either way).  us, 32 / 16 groups:
+    //   16384x5120 12.4 / 12.1, with a gate 23.1 / 19.5
+    //   16384x2624  8.4 /  8.0, with a gate 14.4 / 12.6
+    //   24576x4096 12.7 / 13.1, with a gate 24.9 / 21.9
     const uint32_t tiles = rows / kTileRows;
     const uint32_t groups = cols / kGroup;
-    uint32_t split = std::min<uint32_t>((groups + 31) / 32, 8);
+    // Several vectors stay at 32 groups and six workgroups per CU: each chunk
+    // costs them a meeting per vector (5120x5120, four vectors: 9.9 us in
+    // three chunks, 11.1 in five; 28672x8192 in six and more per CU: 47.6, 50.5).
+    const uint32_t by32 = (groups + 31) / 32, by16 = (groups + 15) / 16;
+    uint32_t split = std::min<uint32_t>(by32, 8);
+    if (vectors == 1 && by16 <= 8 && (by16 < 2 * by32 || (streams > 1 && static_cast<uint64_t>(tiles) * by16 > 6ull * cus))) split = by16;
     if (static_cast<uint64_t>(tiles) * split * 4 < cus)
         split = std::min((cus / 4 + tiles - 1) / tiles, std::max<uint32_t>(1, groups / 16));
-    if (static_cast<uint64_t>(tiles) * split > 6ull * cus) split = std::max<uint32_t>(1, 6 * cus / tiles);
+    // Tall matrices: up to 32 workgroups per CU of such chunks run ahead of
+    // fewer, longer ones (28672x8192 24.0 us in 3584 workgroups against 30.1
+    // in 896, 65536x8192 49.5 in 8192 against 57.2 in 2048); beyond that, or
+    // where chunks hold more than 32 groups anyway, about six per CU.
+    const uint64_t most = vectors > 1 || groups > 32 * split ? 6ull * cus : 32ull * cus;
+    if (static_cast<uint64_t>(tiles) * split > most) split = std::max<uint32_t>(1, 6 * cus / tiles);
     split = std::min(split, std::min(groups, kMaxSplit));
     return std::max<uint32_t>(split, 1);
 }

@@ -161,12 +161,12 @@ uint32_t next_clock_slot() {
 
 bool aligned(const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
-uint32_t policy_split(uint32_t rows, uint32_t cols, int device) {
-    return q4rdna::host::policy_split(rows, cols, cu_count(device));
+uint32_t policy_split(uint32_t rows, uint32_t cols, int device, uint32_t streams = 1, uint32_t vectors = 1) {
+    return q4rdna::host::policy_split(rows, cols, cu_count(device), streams, vectors);
 }
 
-uint32_t resolve_split(const q4rdna_weight *w, uint32_t split) {
-    if (split == 0) split = policy_split(w->rows, w->columns, w->device);
+uint32_t resolve_split(const q4rdna_weight *w, uint32_t split, uint32_t streams) {
+    if (split == 0) split = policy_split(w->rows, w->columns, w->device, streams);
     split = std::min(split, w->columns / kGroup);
     split = std::min(split, kMaxSplit);
     return std::max<uint32_t>(split, 1);
@@ -255,7 +255,7 @@ int check_mul_mat_ex(const q4rdna_weight *w, const q4rdna_weight *gate, const fl
         *launch = L;
         return Q4RDNA_OK;
     }
-    L.split = resolve_split(w, s);
+    L.split = resolve_split(w, s, gate ? 2 : 1);
     if (!gemv_shape_fits(w->rows / kTileRows, w->columns / kGroup, L.split))
         return set_error(Q4RDNA_ERR_ARGUMENT, "shape %ux%u at split %u is beyond the kernels' index range", w->rows,
                          w->columns, L.split);
@@ -783,7 +783,7 @@ int q4rdna_mul_mat_batch(const q4rdna_weight *w, const q4rdna_weight *gate, cons
         count_launch(w->tiles, gt, n);
         return Q4RDNA_OK;
     }
-    if (split == 0) split = policy_split(w->rows, w->columns, w->device);
+    if (split == 0) split = policy_split(w->rows, w->columns, w->device, 1, n);
     split = std::min(std::max(split, need), std::min(groups, kMaxSplit));
     q4rdna::GemvArgs args{};
     args.w = w->tiles;
