@@ -127,7 +127,9 @@ int q4rdna_scope_allows(const char *scope, const char *name);
  * Launches with split K use a scratch buffer per (device, stream).  The
  * first call that needs more than the stream has allocates it (and waits
  * for the device), so it cannot run under HIP graph capture: make one call
- * of each shape on the stream before capturing.  Outgrown buffers are
+ * of each shape on the stream before capturing.  (A policy-chosen split of
+ * a tall matrix, captured without that call, takes fewer chunks instead; it
+ * is refused only where these need a larger buffer too.)  Outgrown buffers are
  * never freed, so a graph captured earlier stays valid.  Calls on one
  * stream are ordered by it; a graph must not replay on another stream
  * while the stream it was captured on runs such calls.

@@ -70,7 +70,7 @@ extern "C" int q4rdna_mul_mat_ex_noalloc(const q4rdna_weight *w, const q4rdna_we
     const uint8_t *gt = gate ? gate->tiles : nullptr;
     // The policy's split is a choice: a tall matrix whose chunks would need
     // more slots than there are takes fewer.
-    if (options == nullptr || options->split_k == 0) {
+    if (L.by_policy) {
         while (L.slots > Q4RDNA_NOALLOC_SLOTS) {
             L.split /= 2;
             L.slots = L.split < 2 ? 0 : static_cast<size_t>(q4rdna::host::exchange_nodes(L.split)) * w->rows * (gate ? 2 : 1);

@@ -172,9 +172,36 @@ uint32_t resolve_split(const q4rdna_weight *w, uint32_t split, uint32_t streams)
     return std::max<uint32_t>(split, 1);
 }
 
-// Per-tensor launch with the stream's split-K workspace.
-int launch_one(const q4rdna::TensorLaunch &launch, const q4rdna_weight *w, const uint8_t *gate, const float *x,
+// Whether the stream is being captured while its workspace is too small for
+// `slots`: a workspace cannot grow there.
+bool captured_without_room(int device, hipStream_t stream, size_t slots) {
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        const auto it = g_ws.find({device, stream});
+        if (it != g_ws.end() && it->second.slot_count >= slots) return false;
+    }
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return status == hipStreamCaptureStatusActive;
+}
+
+// Per-tensor launch with the stream's split-K workspace.  Under capture and
+// without room for the policy's chunks, the policy's choice falls back to
+// the several-vector rule's, whose fewer chunks of a tall matrix often need
+// no workspace.
+int launch_one(const q4rdna::TensorLaunch &wanted, const q4rdna_weight *w, const uint8_t *gate, const float *x,
                const float *add, float *y, hipStream_t stream) {
+    q4rdna::TensorLaunch launch = wanted;
+    if (launch.by_policy && launch.slots > 0 && captured_without_room(w->device, stream, launch.slots)) {
+        const uint32_t split = std::min(policy_split(w->rows, w->columns, w->device, 1, 2), launch.split);
+        if (q4rdna::gemv_shape_fits(w->rows / kTileRows, w->columns / kGroup, split)) {
+            launch.split = split;
+            launch.slots = static_cast<size_t>(q4rdna::host::exchange_nodes(split)) * w->rows * (gate ? 2 : 1);
+        }
+    }
     uint32_t *slots = nullptr;
     if (launch.slots > 0) {
         Workspace *ws = nullptr;
@@ -256,6 +283,7 @@ int check_mul_mat_ex(const q4rdna_weight *w, const q4rdna_weight *gate, const fl
         return Q4RDNA_OK;
     }
     L.split = resolve_split(w, s, gate ? 2 : 1);
+    L.by_policy = s == 0;
     if (!gemv_shape_fits(w->rows / kTileRows, w->columns / kGroup, L.split))
         return set_error(Q4RDNA_ERR_ARGUMENT, "shape %ux%u at split %u is beyond the kernels' index range", w->rows,
                          w->columns, L.split);

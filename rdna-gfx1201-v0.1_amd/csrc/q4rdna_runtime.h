@@ -20,6 +20,7 @@ struct TensorLaunch {
     uint32_t split;
     size_t slots;
     bool sequential;  // Q4RDNA_KERNEL_SEQUENTIAL: split 1, no workspace
+    bool by_policy;   // split is the shape policy's, not the caller's
 };
 
 // Validate q4rdna_mul_mat_ex's arguments (the same statuses as that entry
