@@ -128,11 +128,12 @@ int q4rdna_scope_allows(const char *scope, const char *name);
  * first call that needs more than the stream has allocates it (and waits
  * for the device), so it cannot run under HIP graph capture: make one call
  * of each shape on the stream before capturing.  (A policy-chosen split of
- * a tall matrix, captured without that call, takes fewer chunks instead; it
- * is refused only where these need a larger buffer too.)  Outgrown buffers are
- * never freed, so a graph captured earlier stays valid.  Calls on one
- * stream are ordered by it; a graph must not replay on another stream
- * while the stream it was captured on runs such calls.
+ * a tall matrix or group, captured without that call, takes fewer chunks
+ * instead, so another order of each row's sum and other last bits than the
+ * eager call's; it is refused only where these need a larger buffer too.)
+ * Outgrown buffers are never freed, so a graph captured earlier stays
+ * valid.  Calls on one stream are ordered by it; a graph must not replay on
+ * another stream while the stream it was captured on runs such calls.
  *
  * Replaces ggml_cuda_q4rdna_mul_mat (source/q4rdna.cuh:5-9, q4rdna.cu:713-745). */
 int q4rdna_mul_mat(const q4rdna_weight *w, const float *x, int64_t x_ne0, float *y, int64_t y_ne0,

@@ -188,19 +188,20 @@ bool captured_without_room(int device, hipStream_t stream, size_t slots) {
     return status == hipStreamCaptureStatusActive;
 }
 
+size_t exchange_slots(uint32_t split, size_t rows, uint32_t streams) {
+    return q4rdna::host::exchange_nodes(split) * rows * streams;
+}
+
 // Per-tensor launch with the stream's split-K workspace.  Under capture and
 // without room for the policy's chunks, the policy's choice falls back to
 // the several-vector rule's, whose fewer chunks of a tall matrix often need
-// no workspace.
+// no workspace (launch_group_valu does the same).
 int launch_one(const q4rdna::TensorLaunch &wanted, const q4rdna_weight *w, const uint8_t *gate, const float *x,
                const float *add, float *y, hipStream_t stream) {
     q4rdna::TensorLaunch launch = wanted;
     if (launch.by_policy && launch.slots > 0 && captured_without_room(w->device, stream, launch.slots)) {
-        const uint32_t split = std::min(policy_split(w->rows, w->columns, w->device, 1, 2), launch.split);
-        if (q4rdna::gemv_shape_fits(w->rows / kTileRows, w->columns / kGroup, split)) {
-            launch.split = split;
-            launch.slots = static_cast<size_t>(q4rdna::host::exchange_nodes(split)) * w->rows * (gate ? 2 : 1);
-        }
+        launch.split = std::min(policy_split(w->rows, w->columns, w->device, 1, 2), launch.split);
+        launch.slots = exchange_slots(launch.split, w->rows, gate ? 2 : 1);
     }
     uint32_t *slots = nullptr;
     if (launch.slots > 0) {
@@ -287,7 +288,7 @@ int check_mul_mat_ex(const q4rdna_weight *w, const q4rdna_weight *gate, const fl
     if (!gemv_shape_fits(w->rows / kTileRows, w->columns / kGroup, L.split))
         return set_error(Q4RDNA_ERR_ARGUMENT, "shape %ux%u at split %u is beyond the kernels' index range", w->rows,
                          w->columns, L.split);
-    L.slots = static_cast<size_t>(host::exchange_nodes(L.split)) * w->rows * (gate ? 2 : 1);
+    L.slots = exchange_slots(L.split, w->rows, gate ? 2 : 1);
     *launch = L;
     return Q4RDNA_OK;
 }
@@ -672,9 +673,13 @@ int launch_group_valu(const q4rdna_group_desc *descs, uint32_t count, const floa
     uint64_t total_rows = 0;
     for (uint32_t i = 0; i < count; ++i) total_rows += descs[i].weight.rows;
     if (total_rows > 0x7fffffffull) return set_error(Q4RDNA_ERR_ARGUMENT, "group too large");
-    uint32_t split = split_k != 0 ? split_k : policy_split(static_cast<uint32_t>(total_rows), cols, device);
-    split = std::max(split, (groups + kGroupChunkGroups - 1) / kGroupChunkGroups);
+    const uint32_t all_rows = static_cast<uint32_t>(total_rows), streams = glu ? 2u : 1u;
+    const uint32_t least = (groups + kGroupChunkGroups - 1) / kGroupChunkGroups;
+    uint32_t split = std::max(split_k != 0 ? split_k : policy_split(all_rows, cols, device), least);
     split = std::min(split, groups);
+    if (split_k == 0 && split > least &&
+        captured_without_room(device, stream, exchange_slots(split, all_rows, streams)))
+        split = std::min(split, std::max(policy_split(all_rows, cols, device, 1, 2), least));
     if (split > kMaxSplit)
         return set_error(Q4RDNA_NOT_APPLICABLE, "K = %u needs more than %u chunks of %u groups", cols, kMaxSplit,
                          kGroupChunkGroups);
@@ -682,15 +687,9 @@ int launch_group_valu(const q4rdna_group_desc *descs, uint32_t count, const floa
     const uint64_t workgroups = static_cast<uint64_t>(tiles) * split;
     if (workgroups > 0x7fffffffull || !q4rdna::gemv_shape_fits(tiles, groups, split))
         return set_error(Q4RDNA_ERR_ARGUMENT, "group too large");
-    const uint32_t streams = glu ? 2u : 1u;
-    size_t slots = 0;
-    for (uint32_t i = 0; i < count; ++i) {
-        const uint32_t rows = descs[i].weight.rows;
-        slots += static_cast<size_t>(q4rdna::host::exchange_nodes(split)) * streams * rows;
-    }
     Workspace *ws = nullptr;
     int rc;
-    if (split > 1 && (rc = get_workspace(device, stream, slots, &ws)) != Q4RDNA_OK) return rc;
+    if (split > 1 && (rc = get_workspace(device, stream, exchange_slots(split, all_rows, streams), &ws)) != Q4RDNA_OK) return rc;
     q4rdna::GemvGroupArgs args{};
     args.x = x;
     args.count = count;
@@ -708,7 +707,7 @@ int launch_group_valu(const q4rdna_group_desc *descs, uint32_t count, const floa
         args.g[i] = q4rdna::GemvGroupEntry{d.weight.tiles, d.gate_tiles, d.add, d.y,
                                            split > 1 ? ws->slots + soff : nullptr, rows, tile_begin};
         tile_begin += rows / kTileRows;
-        soff += static_cast<size_t>(q4rdna::host::exchange_nodes(split)) * streams * rows;
+        soff += exchange_slots(split, rows, streams);
     }
     hipError_t e = q4rdna::launch_gemv_group(args, stream);
     if (e != hipSuccess) return hip_fail(e, "group GEMV launch");
