@@ -125,9 +125,9 @@ int q4rdna_scope_allows(const char *scope, const char *name);
  * it (argument errors otherwise).
  *
  * Launches with split K use a scratch buffer per (device, stream).  The
- * first call that needs more than the stream has allocates it (and waits
- * for the device), so it cannot run under HIP graph capture: make one call
- * of each shape on the stream before capturing.  (A policy-chosen split of
+ * first call that needs more than the stream has allocates it, which it
+ * cannot do while that stream is being captured (other streams may be): make
+ * one call of each shape on the stream before capturing.  (A policy-chosen split of
  * a tall matrix or group, captured without that call, takes fewer chunks
  * instead, so another order of each row's sum and other last bits than the
  * eager call's; it is refused only where these need a larger buffer too.)

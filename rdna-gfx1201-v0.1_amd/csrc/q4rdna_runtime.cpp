@@ -124,28 +124,43 @@ std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 // doubles when it grows, so few are ever retired.
 std::vector<Workspace> g_ws_retired;
 
+bool stream_captured(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return status == hipStreamCaptureStatusActive;
+}
+
+// Zero-filled slots for `stream`, which is not being captured.  Other streams
+// may be, by any thread: in the default capture mode a hipMalloc would be
+// refused and would invalidate their captures, and so would waiting for the
+// device.  So the thread allocates in relaxed mode, and the fill is ordered by
+// the stream, before the launch that asked for it.
+hipError_t new_slots(uint32_t **slots, size_t count, hipStream_t stream) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    e = hipMalloc(slots, count * sizeof(uint32_t));
+    if (e == hipSuccess && (e = hipMemsetAsync(*slots, 0, count * sizeof(uint32_t), stream)) != hipSuccess)
+        (void)hipFree(*slots);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return e;
+}
+
 int get_workspace(int device, hipStream_t stream, size_t slots, Workspace **out) {
     std::lock_guard<std::mutex> lock(g_ws_mu);
     Workspace &ws = g_ws[{device, stream}];
     if (ws.slot_count < slots) {
-        const size_t sc = std::max(slots, 2 * ws.slot_count);
-        if (ws.slots != nullptr) {
-            g_ws_retired.push_back(ws);
-            ws = Workspace{};
-        }
-        uint32_t *sl = nullptr;
-        hipError_t e = hipMalloc(&sl, sc * sizeof(uint32_t));
+        if (stream_captured(stream))
+            return set_error(Q4RDNA_ERR_MEMORY, "split-K workspace: it cannot grow while its stream is being captured");
+        Workspace grown;
+        grown.slot_count = std::max(slots, 2 * ws.slot_count);
+        const hipError_t e = new_slots(&grown.slots, grown.slot_count, stream);
         if (e != hipSuccess) return set_error(Q4RDNA_ERR_MEMORY, "split-K workspace: %s", hipGetErrorString(e));
-        // Set once, complete before any launch uses them (launches on
-        // non-blocking streams are not ordered after the null stream).
-        e = hipMemset(sl, 0, sc * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipDeviceSynchronize();
-        if (e != hipSuccess) {
-            (void)hipFree(sl);
-            return hip_fail(e, "hipMemset");
-        }
-        ws.slots = sl;
-        ws.slot_count = sc;
+        if (ws.slots != nullptr) g_ws_retired.push_back(ws);
+        ws = grown;
     }
     *out = &ws;
     return Q4RDNA_OK;
@@ -180,12 +195,7 @@ bool captured_without_room(int device, hipStream_t stream, size_t slots) {
         const auto it = g_ws.find({device, stream});
         if (it != g_ws.end() && it->second.slot_count >= slots) return false;
     }
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return status == hipStreamCaptureStatusActive;
+    return stream_captured(stream);
 }
 
 size_t exchange_slots(uint32_t split, size_t rows, uint32_t streams) {

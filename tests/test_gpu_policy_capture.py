@@ -2,7 +2,8 @@
 a graph as their stream's first call: the capture takes the several-vector
 rule's one chunk (no workspace) instead of growing one, and every replay equals
 that split's eager launch bit for bit.  On a stream that has room the capture
-takes the policy's split."""
+takes the policy's split.  And calls on a stream that is not captured, whose
+workspaces are made while another stream is."""
 import ctypes
 
 import pytest
@@ -72,3 +73,31 @@ def test_first_group_captured(cuda, heights, cols, gated, warm):
         items.append((w, torch.empty(rows, device="cuda"), g if gated else None))
     x = dev_f32(O.gaussian_x(cols, 3))
     check_captured(lambda split: api.mul_mat_group(items, x, split_k=split), [it[1] for it in items], x, warm)
+
+
+def test_workspace_made_while_another_stream_is_captured(cuda):
+    """The first tall call of a stream runs while another stream is captured
+    (in the default mode), and the capture goes on; so it does after a call on
+    the captured stream that is refused for want of room."""
+    rows, cols = 32768, 64 * 33
+    w = api.QWeight.from_tiles(dev_u8(random_tiles(rows, cols, 1)), rows, cols)
+    x = dev_f32(O.gaussian_x(cols, 3))
+    y, want, count = (torch.full((rows,), float("nan"), device="cuda") for _ in range(3))
+    assert api.mul_mat_ex(w, x, want)
+    count.zero_()
+    captured, other = fresh_stream(), fresh_stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        count.add_(1)
+        assert api.mul_mat_ex(w, x, y, stream=other.cuda_stream)
+        with pytest.raises(RuntimeError, match="cannot grow"):
+            api.mul_mat_ex(w, x, y, split_k=2)
+        count.add_(1)
+    other.synchronize()
+    assert torch.equal(y, want)
+    for rep in range(3):
+        with torch.cuda.stream(captured):
+            graph.replay()
+        captured.synchronize()
+        assert (count == 2 * rep + 2).all()
