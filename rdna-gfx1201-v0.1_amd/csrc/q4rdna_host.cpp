@@ -250,14 +250,6 @@ std::vector<uint32_t> deal_items(const std::vector<uint32_t> &cost, const std::v
     return deal;
 }
 
-// Whether a batched sweep claims its items from a queue.  The fixed deal lets
-// the next item's loads cross an item's end, which counts while a workgroup
-// runs few items; over many, up to four vectors gain more from the balance:
-// at N = 2 the 36 layers of Qwen3-8B (share 207 steps) take 620 us with the
-// deal and 598 with the queue, 18 layers 315 and 331, 9 layers 174 and 202.
-// With eight vectors the deal is ahead throughout (667 against 687 us).
-static bool batch_queue(uint32_t n, double share) { return n > 1 && n <= 4 && share > 140.0; }
-
 int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int device, uint32_t cus, PlanLayout *out,
                 std::string *error) {
     if (out == nullptr || (descs == nullptr && count > 0))
@@ -437,31 +429,23 @@ int layout_plan(const q4rdna_gemv_desc *descs, uint32_t count, uint32_t n, int d
     L.table_bytes = groups * (n == 1 ? sizeof(uint64_t) : sizeof(uint32_t));
     L.workgroups = static_cast<uint32_t>(
         std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(cus) * kPlanWorkgroupsPerCu, items)));
-    // After the group table, the items' list: per item its descriptor index
-    // and its index within the descriptor, in item order for a queue; as
-    // dealt to the workgroups, behind the deal's offsets (padded to an even
-    // count), otherwise.
+    // After the group table, the items' deal to the workgroups in the
+    // kernels' form: the offsets (padded to an even count), then per item its
+    // descriptor index and its index within the descriptor.
+    const std::vector<uint32_t> lists = deal_items(item_costs(L), workgroup_weights(L.workgroups, cus));
+    const uint32_t head = (L.workgroups + 2) & ~1u;
+    L.deal.assign(head + 2 * items, 0);
+    std::copy(lists.begin(), lists.begin() + L.workgroups + 1, L.deal.begin());
     std::vector<uint32_t> owner(items);
     for (uint32_t i = 0; i < count; ++i)
         for (uint32_t item = L.descs[i].item_begin; item < L.descs[i + 1].item_begin; ++item) owner[item] = i;
-    auto entry = [&](uint32_t *out, uint32_t item) {
-        out[0] = owner[item];
-        out[1] = item - L.descs[owner[item]].item_begin;
-    };
-    L.queue = batch_queue(n, share);
-    if (L.queue) {
-        L.batch_list.assign(2 * items, 0);
-        for (uint32_t item = 0; item < items; ++item) entry(&L.batch_list[2 * static_cast<size_t>(item)], item);
-    } else {
-        std::vector<uint32_t> &deal = n == 1 ? L.deal : L.batch_list;
-        const std::vector<uint32_t> lists = deal_items(item_costs(L), workgroup_weights(L.workgroups, cus));
-        const uint32_t head = (L.workgroups + 2) & ~1u;
-        deal.assign(head + 2 * items, 0);
-        std::copy(lists.begin(), lists.begin() + L.workgroups + 1, deal.begin());
-        for (uint64_t k = 0; k < items; ++k) entry(&deal[head + 2 * k], lists[L.workgroups + 1 + k]);
+    for (uint64_t k = 0; k < items; ++k) {
+        const uint32_t item = lists[L.workgroups + 1 + k];
+        L.deal[head + 2 * k] = owner[item];
+        L.deal[head + 2 * k + 1] = item - L.descs[owner[item]].item_begin;
     }
     L.deal_off = align256(L.table_off + L.table_bytes);
-    L.tail_off = align256(L.deal_off + (L.deal.size() + L.batch_list.size()) * sizeof(uint32_t));
+    L.tail_off = align256(L.deal_off + L.deal.size() * sizeof(uint32_t));
     L.scratch_bytes = L.tail_off + tail;
     L.table.assign(n == 1 ? groups : (groups + 1) / 2, 0);
     for (uint32_t i = 0; i < count; ++i)

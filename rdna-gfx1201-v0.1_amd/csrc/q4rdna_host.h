@@ -76,7 +76,7 @@ uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus, uint32_t strea
 // aligned:
 //   [0, table_off)                 activation digits (prep_off[i] per GEMV)
 //   [table_off, +table_bytes)      the prep launch's group table
-//   [deal_off, + 4 per word)       single vectors: the item deal; batches: batch_list
+//   [deal_off, +deal.size() * 4)   the item deal
 //   [tail_off, scratch_bytes)      split-K partials and counters
 // descs[i] describes the caller's descriptor order[i] (longest items first),
 // descs[count] is the sentinel; its prep / partial / counters pointers are
@@ -90,18 +90,16 @@ struct PlanLayout {
     std::vector<uint64_t> table;  // group table: activation address per group (single vectors) or
                                   // descriptor index per group, two uint32 per word (batches)
     uint64_t table_off = 0, table_bytes = 0, deal_off = 0, tail_off = 0, scratch_bytes = 0;
-    std::vector<uint32_t> deal;        // single vectors: see launch_plan in q4rdna_internal.h
-    std::vector<uint32_t> batch_list;  // batches: a deal, or with `queue` the items in order (launch_plan_batch)
-    bool queue = false;
+    std::vector<uint32_t> deal;  // see launch_plan in q4rdna_internal.h
 };
 
-// Item costs of a single-vector plan (one per item, in item order).
+// Item costs of a plan (one per item, in item order).
 std::vector<uint32_t> item_costs(const PlanLayout &layout);
 
 // Time per unit of item cost of each of the plan's workgroups (1024 = 1).
 std::vector<uint32_t> workgroup_weights(uint32_t workgroups, uint32_t cus);
 
-// Deal of a single-vector sweep's items to its workgroups.  cost[i] is item
+// Deal of a sweep's items to its workgroups.  cost[i] is item
 // i's weight in the sweep; weight[b] is workgroup b's time per unit of cost.
 // Returns per workgroup the offset of its list (workgroups + 1 offsets) and
 // the lists, each in increasing item order.

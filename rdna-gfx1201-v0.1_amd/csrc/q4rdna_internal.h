@@ -154,10 +154,8 @@ uint32_t gemv_multi_stage_groups(uint32_t vectors);
 // items, dealt to its workgroups by the plan: deal holds workgroups + 1
 // offsets (padded to an even count), then one (descriptor index, item within
 // the descriptor) pair of uint32 per item; workgroup b runs entries
-// [deal[b], deal[b + 1]), in increasing item order.  The batched sweep takes such a deal as
-// its list, or with `queue` claims its items: then list holds the pairs in
-// item order, without offsets, sched is the queue's two zeroed counters,
-// owned by the plan (left zero after every launch), and workgroups <= items.
+// [deal[b], deal[b + 1]), in increasing item order.  Batched plans are dealt
+// the same way.
 hipError_t launch_prep(const float *const *group_x, uint8_t *prep, uint32_t groups, hipStream_t stream);
 // both_streams: some GEMV has per == 1 with a SwiGLU gate (one item streams
 // both weights); plans without such GEMVs run a sweep built without that path.
@@ -181,8 +179,8 @@ constexpr uint32_t kBatchChunkGroups = 192;
 constexpr uint32_t kMinBatchChunkGroups = 32;
 hipError_t launch_prep_batch(const PlanDesc *descs, const uint32_t *owner, uint32_t groups, uint32_t n,
                              hipStream_t stream);
-hipError_t launch_plan_batch(const PlanDesc *descs, const uint32_t *list, bool queue, uint32_t items, uint32_t n,
-                             uint32_t workgroups, uint32_t *sched, hipStream_t stream);
+hipError_t launch_plan_batch(const PlanDesc *descs, const uint32_t *deal, uint32_t n, uint32_t workgroups,
+                             hipStream_t stream);
 constexpr uint32_t kMaxGroup = 8;  // GEMVs of one group launch (Q4RDNA_MAX_GROUP)
 
 // A VALU group launch (gemv_kernel's arithmetic): up to kMaxGroup GEMVs

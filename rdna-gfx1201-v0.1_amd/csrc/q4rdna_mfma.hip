@@ -31,8 +31,6 @@
 //    activation digits are stored in the same order.
 //
 // The sweep kernel's lane mapping is described at the kernel below.
-#include <type_traits>
-
 #include "q4rdna_device.h"
 
 namespace q4rdna {
@@ -982,7 +980,6 @@ constexpr int kBatchWaves = 4;  // eight waves per workgroup measured slower
 // its last step, so the two uses never overlap): 4*NQ x 256 floats <= 8 KB.
 struct BatchShared {
     uint8_t stage[kBatchWaves][kStageBytes];
-    uint3 next_item;  // the next item's number and table entry
     uint32_t last;
 };
 static_assert(8 * kBatchRows * sizeof(float) <= kStageBytes, "partials must fit a wave's stage");
@@ -1093,6 +1090,11 @@ __device__ __forceinline__ void batch_steps(uint8_t *stage, const uint8_t *w, co
             a[vq] = *(gptr_i32x4)(pg + vq * kBatchQuadBytes + 256 * kslot + 16 * j);
             f[vq] = *(gptr_cf32)(pg + vq * kBatchQuadBytes + 1024 + 4 * kslot);
         }
+        // All of a step's loads are issued before it waits for any.  With the
+        // barrier ahead of the digits' loads the compiler left these until the
+        // tiles had arrived, a second round trip per step: 12 / 24 layers of
+        // Qwen3-8B with gates, N = 2, 228 / 421 us instead of 210 / 401.
+        __builtin_amdgcn_sched_barrier(0);
         // Restaged through registers: loading straight into LDS, as the
         // single-vector sweep does, measured neutral to 0.6 % slower here.
 #pragma unroll
@@ -1113,7 +1115,6 @@ __device__ __forceinline__ void batch_steps(uint8_t *stage, const uint8_t *w, co
     for (; g < c.g_end; g += kBatchWaves) {
         BatchRegs r;
         load_batch_step(w, c, g, lane, r);
-        __builtin_amdgcn_sched_barrier(0);
         step(g, r);
     }
 }
@@ -1176,33 +1177,24 @@ __device__ __forceinline__ void finish_batch_item(uint32_t &last, const BatchIte
     if (threadIdx.x == 0) store_agent(&c.counters[c.block], 0u);
 }
 
-// QUEUE: workgroup b runs item b, then items claimed from a queue; list[item]
-// is an item's descriptor and its index within it (walking the GEMVs' item
-// ranges instead cost a dependent load per GEMV passed).  Thread 0 claims two
-// items ahead and reads the next one's entry while an item's steps run, so
-// that neither round trip is waited for.  Otherwise list is a deal, as
-// plan_kernel's, and every wave loads the next item's first step across an
-// item's end.  batch_queue (q4rdna_host.cpp) says which a plan takes.
-template <int NQ, bool QUEUE>
+// Workgroup b runs entries [deal[b], deal[b + 1]) of the plan's deal, as
+// plan_kernel does, and every wave loads the next item's first step across an
+// item's end.
+template <int NQ>
 __global__ __launch_bounds__(64 * kBatchWaves, 2) void plan_batch_kernel(const PlanDesc *__restrict__ descs,
-                                                                         const uint32_t *__restrict__ list, uint32_t items,
-                                                                         uint32_t nvec, uint32_t *__restrict__ sched) {
+                                                                         const uint32_t *__restrict__ deal,
+                                                                         uint32_t nvec) {
     __shared__ BatchShared sh;
     const int lane = threadIdx.x & 63, wave = wave_id();
 #if defined(Q4RDNA_SWEEP_CLOCKS)
     const uint64_t clock_start = __builtin_amdgcn_s_memrealtime();
 #endif
-    const uint2 *entry = reinterpret_cast<const uint2 *>(QUEUE ? list : list + ((gridDim.x + 2) & ~1u));
-    // The item's entry, and the end of the entries that are the workgroup's
-    // (a queued plan launches at most `items` workgroups).
-    uint32_t k = QUEUE ? blockIdx.x : list[blockIdx.x];
-    const uint32_t end = QUEUE ? items : list[blockIdx.x + 1];
+    const uint2 *entry = reinterpret_cast<const uint2 *>(deal + ((gridDim.x + 2) & ~1u));
+    uint32_t k = deal[blockIdx.x];
+    const uint32_t end = deal[blockIdx.x + 1];
     if (k >= end) return;
     auto locate = [&](uint2 e) { return decode_batch_item(descs[e.x], e.y); };
     BatchItem cur = locate(entry[k]);
-    auto claim = [&]() { return gridDim.x + add_agent(&sched[0], 1u); };
-    uint32_t claimed = 0;  // thread 0 of a queued sweep: the next item
-    if (QUEUE && threadIdx.x == 0) claimed = claim();
     BatchRegs pre;
     bool have_pre = false;
     const int kslot = lane >> 4, T = (lane & 15) >> 1, h = lane & 1;
@@ -1227,13 +1219,8 @@ __global__ __launch_bounds__(64 * kBatchWaves, 2) void plan_batch_kernel(const P
         return v;
     };
     for (;;) {
-        uint32_t claimed2 = 0;
         uint2 e = make_uint2(0, 0);
-        if (QUEUE && threadIdx.x == 0) {
-            e = entry[min(claimed, items - 1)];
-            claimed2 = claim();
-        }
-        if (!QUEUE && k + 1 < end) e = entry[k + 1];
+        if (k + 1 < end) e = entry[k + 1];
         float acc[NQ][16], u[4 * NQ];
         auto clear = [&]() {
 #pragma unroll
@@ -1257,12 +1244,7 @@ __global__ __launch_bounds__(64 * kBatchWaves, 2) void plan_batch_kernel(const P
         publish(acc);
         BatchItem next;
         have_pre = false;
-        if constexpr (QUEUE) {
-            if (threadIdx.x == 0) {
-                sh.next_item = make_uint3(claimed, e.x, e.y);
-                claimed = claimed2;
-            }
-        } else if (++k < end) {
+        if (++k < end) {
             next = locate(e);
             if (next.g_begin + wave < next.g_end) {
                 load_batch_step(next.w, next, next.g_begin + wave, lane, pre);
@@ -1270,22 +1252,10 @@ __global__ __launch_bounds__(64 * kBatchWaves, 2) void plan_batch_kernel(const P
             }
         }
         __syncthreads();
-        if constexpr (QUEUE) k = __builtin_amdgcn_readfirstlane(sh.next_item.x);
-        if (QUEUE && k < end)
-            next = locate(make_uint2(__builtin_amdgcn_readfirstlane(sh.next_item.y),
-                                     __builtin_amdgcn_readfirstlane(sh.next_item.z)));
         finish_batch_item<NQ>(sh.last, cur, nvec, total, u);
         if (k >= end) break;
-        __syncthreads();  // the partials and the next item are read
+        __syncthreads();  // the partials are read
         cur = next;
-    }
-    // The last workgroup to end, with every claim made, empties the queue.
-    if (QUEUE && threadIdx.x == 0) {
-        wait_stores();
-        if (add_agent(&sched[1], 1u) == gridDim.x - 1) {
-            store_agent(&sched[0], 0u);
-            store_agent(&sched[1], 0u);
-        }
     }
 #if defined(Q4RDNA_SWEEP_CLOCKS)
     __syncthreads();
@@ -1349,22 +1319,13 @@ hipError_t launch_prep_batch(const PlanDesc *descs, const uint32_t *owner, uint3
     return hipGetLastError();
 }
 
-hipError_t launch_plan_batch(const PlanDesc *descs, const uint32_t *list, bool queue, uint32_t items, uint32_t n,
-                             uint32_t workgroups, uint32_t *sched, hipStream_t stream) {
-    const dim3 grid(workgroups), block(64 * kBatchWaves);
-    auto go = [&](auto nq, auto q) {
-        hipLaunchKernelGGL((plan_batch_kernel<decltype(nq)::value, decltype(q)::value>), grid, block, 0, stream, descs, list,
-                           items, n, sched);
-    };
-    using One = std::integral_constant<int, 1>;
-    using Two = std::integral_constant<int, 2>;
-    if (n > 4 && queue) return hipErrorInvalidValue;  // batch_queue takes it for one quad only
-    if (n > 4)
-        go(Two{}, std::false_type{});
-    else if (queue)
-        go(One{}, std::true_type{});
+hipError_t launch_plan_batch(const PlanDesc *descs, const uint32_t *deal, uint32_t n, uint32_t workgroups,
+                             hipStream_t stream) {
+    const dim3 block(64 * kBatchWaves);
+    if (n <= 4)
+        hipLaunchKernelGGL(plan_batch_kernel<1>, dim3(workgroups), block, 0, stream, descs, deal, n);
     else
-        go(One{}, std::false_type{});
+        hipLaunchKernelGGL(plan_batch_kernel<2>, dim3(workgroups), block, 0, stream, descs, deal, n);
     return hipGetLastError();
 }
 

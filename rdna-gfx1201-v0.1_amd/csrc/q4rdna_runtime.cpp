@@ -343,15 +343,13 @@ struct q4rdna_plan {
     std::vector<const uint8_t *> weights;  // every GEMV's tiles (and gate tiles): the launch's hits
     q4rdna::PlanDesc *descs = nullptr;  // count + 1 (sentinel)
     uint8_t *scratch = nullptr;         // activation digits, split-K partials and counters
-    uint32_t *sched = nullptr;          // batched sweeps' [next item, finished workgroups], zero between launches
     uint8_t *table = nullptr;           // prep launch's group table (in scratch)
-    uint32_t *deal = nullptr;           // the sweep's item deal or queue list (in scratch)
+    uint32_t *deal = nullptr;           // the sweep's item deal (in scratch)
     uint32_t count = 0;
     uint32_t items = 0;
     uint32_t groups = 0;
     uint32_t workgroups = 0;
     uint32_t batch = 1;  // activation vectors per GEMV
-    bool queue = false;         // a batched sweep that claims its items
     bool both_streams = false;  // some SwiGLU GEMV runs both weight streams in one item
 };
 
@@ -870,7 +868,6 @@ int q4rdna_plan_create_batch(const q4rdna_gemv_desc *descs, uint32_t count, uint
     plan->device = device;
     plan->batch = n;
     plan->both_streams = L.both_streams;
-    plan->queue = L.queue;
     plan->count = count;
     for (uint32_t i = 0; i < count; ++i) {
         plan->weights.push_back(descs[i].weight.tiles);
@@ -882,11 +879,9 @@ int q4rdna_plan_create_batch(const q4rdna_gemv_desc *descs, uint32_t count, uint
     auto cleanup = [&plan]() {
         if (plan->descs) (void)hipFree(plan->descs);
         if (plan->scratch) (void)hipFree(plan->scratch);
-        if (plan->sched) (void)hipFree(plan->sched);
     };
     hipError_t e = hipMalloc(&plan->descs, L.descs.size() * sizeof(q4rdna::PlanDesc));
     if (e == hipSuccess && L.scratch_bytes > 0) e = hipMalloc(&plan->scratch, L.scratch_bytes);
-    if (e == hipSuccess) e = hipMalloc(&plan->sched, 2 * sizeof(uint32_t));
     if (e != hipSuccess) {
         cleanup();
         return set_error(Q4RDNA_ERR_MEMORY, "plan buffers: %s", hipGetErrorString(e));
@@ -903,10 +898,8 @@ int q4rdna_plan_create_batch(const q4rdna_gemv_desc *descs, uint32_t count, uint
     e = hipMemcpy(plan->descs, L.descs.data(), L.descs.size() * sizeof(q4rdna::PlanDesc), hipMemcpyHostToDevice);
     if (e == hipSuccess && L.scratch_bytes > 0) e = hipMemset(plan->scratch, 0, L.scratch_bytes);
     if (e == hipSuccess && L.groups > 0) e = hipMemcpy(plan->table, L.table.data(), L.table_bytes, hipMemcpyHostToDevice);
-    const std::vector<uint32_t> &entries = n == 1 ? L.deal : L.batch_list;
-    if (e == hipSuccess && !entries.empty())
-        e = hipMemcpy(plan->deal, entries.data(), entries.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(plan->sched, 0, 2 * sizeof(uint32_t));
+    if (e == hipSuccess && !L.deal.empty())
+        e = hipMemcpy(plan->deal, L.deal.data(), L.deal.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
         cleanup();
@@ -947,8 +940,8 @@ int q4rdna_plan_sweep(q4rdna_plan *plan, void *stream) {
     hipError_t e = plan->batch == 1
                        ? q4rdna::launch_plan(plan->descs, plan->deal, plan->workgroups, plan->both_streams,
                                              static_cast<hipStream_t>(stream))
-                       : q4rdna::launch_plan_batch(plan->descs, plan->deal, plan->queue, plan->items, plan->batch,
-                                                   plan->workgroups, plan->sched, static_cast<hipStream_t>(stream));
+                       : q4rdna::launch_plan_batch(plan->descs, plan->deal, plan->batch, plan->workgroups,
+                                                   static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "plan sweep launch");
     count_launch(plan->weights.data(), plan->weights.size());
     return Q4RDNA_OK;
@@ -965,7 +958,6 @@ void q4rdna_plan_destroy(q4rdna_plan *plan) {
     DeviceGuard guard(plan->device);
     if (plan->descs != nullptr) (void)hipFree(plan->descs);
     if (plan->scratch != nullptr) (void)hipFree(plan->scratch);
-    if (plan->sched != nullptr) (void)hipFree(plan->sched);
     delete plan;
 }
 

@@ -63,9 +63,9 @@ std::vector<q4rdna_gemv_desc> make_descs(const std::vector<Shape> &shapes, uint3
     return d;
 }
 
-std::vector<Shape> qwen3_stack(bool fused) {
+std::vector<Shape> qwen3_stack(bool fused, int layers = 36) {
     std::vector<Shape> s;
-    for (int layer = 0; layer < 36; ++layer) {
+    for (int layer = 0; layer < layers; ++layer) {
         s.push_back({4096, 4096, false, false});   // q
         s.push_back({1024, 4096, false, false});   // k
         s.push_back({1024, 4096, false, false});   // v
@@ -120,8 +120,21 @@ void check_layout(const std::string &name, const std::vector<Shape> &shapes, uin
         expect(p.prep == nullptr && p.partial == nullptr && p.counters == nullptr, "pointers unbased", name);
         expect(L.prep_off[i] == groups * (n == 1 ? q4rdna::kPrepBytes : (n + 3) / 4 * q4rdna::kBatchQuadBytesHost),
                "prep offset", name);
+        // The K chunks cover the row, none is empty; one item per block with
+        // both streams or two blocks in one item, else one per stream and chunk.
+        const uint32_t row_groups = p.cols / 64, streams = d.gate_tiles != nullptr ? 2u : 1u;
+        expect(p.chunk_groups >= 1 && (p.chunks - 1) * p.chunk_groups < row_groups &&
+                   p.chunks * p.chunk_groups >= row_groups,
+               "chunks cover the row", name);
+        expect(p.chunk_groups <= (n == 1 ? q4rdna::kChunkGroups : q4rdna::kBatchChunkGroups), "chunk length", name);
+        expect(p.streams == streams, "streams", name);
+        expect(p.per == p.chunks * streams || (p.per == 1 && p.chunks == 1), "items per block", name);
+        const uint32_t item_rows = (n == 1 ? q4rdna::kBlockRows : q4rdna::kBatchBlockRows) * (p.pair ? 2 : 1);
+        expect(!p.pair || (n == 1 && streams == 1 && p.per == 1), "pairs", name);
+        expect(L.descs[i + 1].item_begin - p.item_begin == (p.rows + item_rows - 1) / item_rows * p.per, "item count",
+               name);
         items = L.descs[i + 1].item_begin;
-        groups += p.cols / 64;
+        groups += row_groups;
         per_one &= p.per == 1;
         if (p.per > 1) {
             expect(align_check(L.part_off[i]) == 0 && align_check(L.cnt_off[i]) == 0, "tail alignment", name);
@@ -151,7 +164,7 @@ void check_layout(const std::string &name, const std::vector<Shape> &shapes, uin
                 expect(reinterpret_cast<const uint32_t *>(L.table.data())[g] == i, "group table owner", name);
         }
     double max_load = 0.0, mean_load = 0.0;
-    if (n == 1) {
+    {
         // The deal: offsets, then (descriptor, item within it) pairs; every
         // item exactly once, each workgroup's list ascending.
         const uint32_t W = L.workgroups, head = (W + 2) & ~1u;
@@ -179,8 +192,6 @@ void check_layout(const std::string &name, const std::vector<Shape> &shapes, uin
             mean_load += static_cast<double>(load) / W;
         }
         for (uint32_t i = 0; i < L.items; ++i) expect(dealt[i] == 1, "every item dealt once", name);
-    } else {
-        expect(L.deal.empty(), "batched plans have no deal", name);
     }
     std::printf("{\"plan\": \"%s\", \"gemvs\": %u, \"batch\": %u, \"items\": %u, \"groups\": %u, \"workgroups\": %u, "
                 "\"scratch_bytes\": %llu, \"all_per_one\": %s, \"both_streams\": %s, \"max_load\": %.0f, "
@@ -196,6 +207,15 @@ int run_layout() {
     check_layout("qwen3_252_batch4", qwen3_stack(false), 4, 256);
     check_layout("qwen3_252_batch8", qwen3_stack(false), 8, 256);
     check_layout("qwen3_216_swiglu_batch8", qwen3_stack(true), 8, 256);
+    // Batches with little work per workgroup: rows in K chunks, streams apart.
+    for (uint32_t n : {2u, 8u}) {
+        check_layout("qwen3_1_layer_swiglu_batch" + std::to_string(n), qwen3_stack(true, 1), n, 256);
+        check_layout("qwen3_5_layers_swiglu_batch" + std::to_string(n), qwen3_stack(true, 5), n, 256);
+        check_layout("few_items_batch" + std::to_string(n),
+                     {{288, 2624, false, false}, {512, 4096, true, true}, {256, 12480, false, true}, {32, 64, false, false}},
+                     n, 256);
+    }
+    check_layout("many_items_batch3", std::vector<Shape>(5120, {256, 4096, false, false}), 3, 256);
     check_layout("mixed", mixed_plan(7), 1, 256);
     check_layout("mixed_batch3", mixed_plan(8), 3, 256);
     check_layout("mixed_small_gpu", mixed_plan(9), 1, 8);

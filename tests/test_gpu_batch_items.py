@@ -1,6 +1,6 @@
 """Batched plans at the sizes where their items change: plans of little work
 (rows cut into K chunks, streams and chunks meeting in memory), of more
-(whole rows, a deal), and of enough for the item queue, at one and two vector
+(whole rows), and of many items per workgroup, at one and two vector
 quads.  Every vector against both parity bars."""
 import numpy as np
 import pytest
@@ -34,7 +34,7 @@ def test_batched_items(cuda, n, repeat):
         items += [(args[0], args[1], y, args[2], args[3]) for y in ys]
         want.append((t, rows, cols, xs, gt, add, ys))
     plan = api.Plan(items, batch=n)
-    for _ in range(2):  # the second launch finds the counters and the queue as the first left them
+    for _ in range(2):  # the second launch finds the counters as the first left them
         for it in items:
             it[2].fill_(float("nan"))
         assert plan.launch()
@@ -50,7 +50,7 @@ def test_batched_items(cuda, n, repeat):
 
 
 def test_batched_queue(cuda):
-    """More than 140 steps per workgroup: the queue, over several launches."""
+    """Ten items of 16 steps per workgroup, over several launches."""
     rows, cols, n = 256, 4096, 3
     t = random_tiles(rows, cols, 3400)
     w = api.QWeight.from_tiles(dev_u8(t), rows, cols)

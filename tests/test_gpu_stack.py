@@ -329,8 +329,8 @@ def test_plan_with_many_items_per_workgroup(cuda):
 
 
 def test_batched_plan_with_many_items(cuda):
-    """The batched sweep's queue with more items than workgroups (three
-    vectors per GEMV): every vector of every GEMV against both bars."""
+    """The batched sweep with more items than workgroups (three vectors per
+    GEMV): every vector of every GEMV against both bars."""
     gemvs = make_gemvs(3, 4)
     ys, wg = run_plan(gemvs, 3)
     assert len(gemvs) > wg

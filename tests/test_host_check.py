@@ -53,6 +53,15 @@ def test_plan_layout_and_deal_under_sanitizers(host_check):
     # (up and gate in one item), down 16: 104 items per layer, no partials.
     g8 = by["qwen3_216_swiglu_batch8"]
     assert g8["gemvs"] == 216 and g8["all_per_one"] and g8["both_streams"] and g8["items"] == 104 * 36
+    # Batches with little work cut rows into chunks and SwiGLU sites into streams.
+    for n in (2, 8):
+        assert not by[f"qwen3_1_layer_swiglu_batch{n}"]["all_per_one"]
+        assert not by[f"few_items_batch{n}"]["all_per_one"]
+        assert by[f"qwen3_5_layers_swiglu_batch{n}"]["workgroups"] == 512
+    # Batches are dealt as evenly as their items allow (here ten each).
+    many = by["many_items_batch3"]
+    assert (many["items"], many["workgroups"]) == (5120, 512) and many["max_load"] <= 1.1 * many["mean_load"]
+    assert by["qwen3_252_batch4"]["max_load"] <= 1.15 * by["qwen3_252_batch4"]["mean_load"]
     assert not by["mixed"]["all_per_one"] and by["mixed"]["both_streams"]
     assert by["mixed_small_gpu"]["workgroups"] == 16
     assert by["one_gemv"]["items"] == 1
