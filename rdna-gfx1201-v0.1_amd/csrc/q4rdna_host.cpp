@@ -71,40 +71,84 @@ bool valid_shape(uint32_t rows, uint32_t cols) {
     return rows > 0 && cols > 0 && rows % kTileRows == 0 && cols % kGroup == 0;
 }
 
-uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus, uint32_t streams, uint32_t vectors) {
-    // About 32 groups per workgroup (eight waves of four tiles, all in flight
-    // at once) and at most 8 chunks; more chunks only when the row tiles are
-    // so few that under a quarter of the CUs would get a workgroup.  Measured
-    // on MI355X (split sweep, with and without a SwiGLU gate): 4096x4096 best
-    // at 2, 1024x4096 at 2-4, 12288x4096 at 2, 4096x12288 at 6, 2048x28672 at
-    // 7-8, 151936x4096 at 1-2.
-    //
-    // A wave holds 1, 2, 4 or 8 tiles, so 16 groups per workgroup are taken
-    // where they fill the waves better than 32 (41 groups: three chunks of 14
-    // instead of two of 21), and with a gate, whose chunks are twice the
-    // bytes, once that makes more than six workgroups per CU (12288x4096 with
-    // a gate, six, measures 12.5 us either way).  us, 32 / 16 groups:
-    //   16384x5120 12.4 / 12.1, with a gate 23.1 / 19.5
-    //   16384x2624  8.4 /  8.0, with a gate 14.4 / 12.6
-    //   24576x4096 12.7 / 13.1, with a gate 24.9 / 21.9
-    const uint32_t tiles = rows / kTileRows;
-    const uint32_t groups = cols / kGroup;
-    // Several vectors stay at 32 groups and six workgroups per CU: each chunk
-    // costs them a meeting per vector (5120x5120, four vectors: 9.9 us in
-    // three chunks, 11.1 in five; 28672x8192 in six and more per CU: 47.6, 50.5).
-    const uint32_t by32 = (groups + 31) / 32, by16 = (groups + 15) / 16;
-    uint32_t split = std::min<uint32_t>(by32, 8);
-    if (vectors == 1 && by16 <= 8 && (by16 < 2 * by32 || (streams > 1 && static_cast<uint64_t>(tiles) * by16 > 6ull * cus))) split = by16;
+// About 32 groups per workgroup (eight waves of four tiles, all in flight at
+// once) and at most 8 chunks; more chunks only when the row tiles are so few
+// that under a quarter of the CUs would get a workgroup, fewer when there would
+// be more than six workgroups per CU.  Measured on MI355X (split sweep, with
+// and without a SwiGLU gate): 4096x4096 best at 2, 1024x4096 at 2-4, 12288x4096
+// at 2, 4096x12288 at 6, 2048x28672 at 7-8, 151936x4096 at 1-2.
+static uint32_t coarse_split(uint32_t tiles, uint32_t groups, uint32_t cus) {
+    uint32_t split = std::min<uint32_t>((groups + 31) / 32, 8);
     if (static_cast<uint64_t>(tiles) * split * 4 < cus)
         split = std::min((cus / 4 + tiles - 1) / tiles, std::max<uint32_t>(1, groups / 16));
-    // Tall matrices: up to 32 workgroups per CU of such chunks run ahead of
-    // fewer, longer ones (28672x8192 24.0 us in 3584 workgroups against 30.1
-    // in 896, 65536x8192 49.5 in 8192 against 57.2 in 2048); beyond that, or
-    // where chunks hold more than 32 groups anyway, about six per CU.
-    const uint64_t most = vectors > 1 || groups > 32 * split ? 6ull * cus : 32ull * cus;
-    if (static_cast<uint64_t>(tiles) * split > most) split = std::max<uint32_t>(1, 6 * cus / tiles);
-    split = std::min(split, std::min(groups, kMaxSplit));
-    return std::max<uint32_t>(split, 1);
+    if (static_cast<uint64_t>(tiles) * split > 6ull * cus) split = 6 * cus / tiles;
+    return std::max<uint32_t>(1, std::min(split, std::min(groups, kMaxSplit)));
+}
+
+// The finer of two splits where it is the faster one, of about 900 timings of
+// both (8 to 3072 row tiles, 33 to 256 groups, with and without a gate, single
+// launches and groups; us in the lines below are single launches, coarse /
+// fine).
+uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus, bool gate, LaunchKind kind) {
+    const uint32_t tiles = rows / kTileRows, groups = cols / kGroup;
+    const uint32_t coarse = coarse_split(tiles, groups, cus);
+    // Several vectors: each chunk costs a meeting per vector (5120x5120, four
+    // vectors: 9.9 us in three chunks, 11.1 in five; 28672x8192 47.6, 50.5).
+    if (kind == LaunchKind::kVectors) return coarse;
+    auto wgs = [&](uint32_t split) { return static_cast<uint64_t>(tiles) * split; };
+
+    // Chunks of about 16 groups where they fill the waves, which hold 1, 2, 4
+    // or 8 tiles, better than 32 (41 groups: three chunks of 14 instead of two
+    // of 21), and in single launches with a gate, whose chunks are twice the
+    // bytes, once that makes more than six workgroups per CU (12288x4096 with
+    // a gate, six, measures 12.5 either way; 16384x4096 15.4 / 15.2, 22400x4096
+    // 22.5 / 19.6).
+    const uint32_t by32 = (groups + 31) / 32, by16 = (groups + 15) / 16;
+    const bool finer = by16 <= 8 && (by16 < 2 * by32 || (gate && kind == LaunchKind::kSingle && wgs(by16) > 6ull * cus));
+    const uint32_t fine = finer ? by16 : std::min<uint32_t>(by32, 8);
+    // Long rows (chunks of more than 32 groups at eight chunks) stay at six
+    // workgroups per CU.  So does what would pass 32 per CU: 65536x8192, 32 per
+    // CU, 55.3 / 47.9, but nothing finer is tried beyond (65568x8192 in one
+    // chunk 55.3, in two 50.3; 64000x5120 in one 36.8, in three 33.1).
+    if (fine == coarse || groups > 32 * fine || wgs(fine) * 4 < cus || wgs(fine) > 32ull * cus) return coarse;
+
+    // The groups of the CU with the most workgroups.
+    auto fullest = [&](uint32_t split) { return (wgs(split) + cus - 1) / cus * ((groups + split - 1) / split); };
+    if (coarse >= by32) {
+        // 16 groups against 32.  Without a gate a launch of at most one
+        // workgroup per CU is latency that more chunks only add to (3072x2624
+        // 4.07 / 4.49); with more it depends on the fullest CU (5120x2624, 42
+        // groups / 28, 4.88 / 4.64; 5120x4608, 48 / 60, 5.88 / 6.18), past two
+        // chunks only a clear gain there shows (4096x4160, 44 / 39, 5.46 /
+        // 5.66; 6144x4160, 66 / 52, 6.50 / 6.23), and from four per CU on the
+        // finer chunks win (12288x5120 10.02 / 9.53), groups' where the fullest
+        // CU has no more to do (12288x7168, 168 / 176, 11.90 / 12.43).
+        if (!gate && wgs(by32) < 4ull * cus)
+            return wgs(by32) > cus && (by32 == 2 ? fullest(fine) <= fullest(coarse)
+                                                 : 100 * fullest(fine) < 87 * fullest(coarse))
+                       ? fine : coarse;
+        if (!gate && kind == LaunchKind::kGroup && by32 > 2 && fullest(fine) > fullest(coarse)) return coarse;
+        // With a gate they win unless the fullest CU gets much more to do
+        // (2720x4608, 24 / 30 groups, 6.49 / 6.65; 5120x4160, 44 / 52, 8.57 /
+        // 8.91; 6144x6208, 75 / 84, 12.06 / 11.77).
+        return !gate || by32 <= 2 || by16 == 2 * by32 || 8 * fullest(fine) <= 9 * fullest(coarse) ? fine : coarse;
+    }
+    // Tall matrices: up to 32 workgroups per CU of short chunks run ahead of
+    // six of longer ones (28672x8192 27.5 / 23.5, 9216x16384 20.6 / 17.3;
+    // 32768x2624 with a gate 24.9 / 19.7).  Coarse chunks of more than 64
+    // groups, which only single launches run, go through the pipelined loop,
+    // which pads nothing: against it 16-group chunks must fill their waves
+    // (32768x4160, 13 of 16, 16.6 / 17.7; 32768x6208, 14, 23.1 / 23.4;
+    // 49152x4608, 15, 25.3 / 25.5; 32768x5120, 16, 19.9 / 18.9), and 32-group
+    // chunks with a gate (32768x8256, 26 of 32, 53.8 / 59.4; 12800x12352, 28,
+    // 35.2 / 37.6; 12800x14400, 29, 42.6 / 41.6).
+    // One chunk of a group with a gate, of up to 64 groups, is not cut into
+    // 32-group ones (49152x4096 39.6 / 41.6).
+    if (gate && !finer && groups <= 64 && coarse == 1) return coarse;
+    if (kind == LaunchKind::kSingle && groups > 64 * coarse) {
+        if (finer ? 100 * groups < 83 * 16 * fine : gate && 8 * groups < 7 * 32 * fine) return coarse;
+    }
+    return fine;
 }
 
 // Steps of 32 tiles of an item that makes `passes` passes over its groups.

@@ -66,10 +66,14 @@ constexpr uint32_t kMaxSplit = 64;
 // without a split.
 constexpr uint32_t exchange_nodes(uint32_t split) { return exchange_leaves(split) - 1; }
 
-// Split-K factor of a per-tensor launch of rows x cols on a GPU with `cus`
-// compute units that streams one weight, or two (a SwiGLU gate too), for
-// `vectors` activation vectors.
-uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus, uint32_t streams, uint32_t vectors);
+// Launches that ask the shape policy: one GEMV, a group of GEMVs on one
+// activation (rows are all of them together; no chunk over kGroupChunkGroups
+// groups), one GEMV on several vectors.
+enum class LaunchKind { kSingle, kGroup, kVectors };
+
+// Split-K factor of a launch of rows x cols on a GPU with `cus` compute units,
+// with a SwiGLU gate or without.
+uint32_t policy_split(uint32_t rows, uint32_t cols, uint32_t cus, bool gate, LaunchKind kind);
 
 // Everything a plan is made of, computed on the host.  Scratch regions are
 // byte offsets from the start of the plan's scratch buffer, all 256-byte

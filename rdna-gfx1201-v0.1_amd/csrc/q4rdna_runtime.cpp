@@ -55,6 +55,7 @@ using q4rdna::host::Entry;
 using q4rdna::host::FileEntry;
 using q4rdna::host::FileHeader;
 using q4rdna::host::kMaxSplit;
+using q4rdna::host::LaunchKind;
 using q4rdna::host::valid_shape;
 
 int hip_fail(hipError_t e, const char *what) {
@@ -176,12 +177,12 @@ uint32_t next_clock_slot() {
 
 bool aligned(const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
-uint32_t policy_split(uint32_t rows, uint32_t cols, int device, uint32_t streams = 1, uint32_t vectors = 1) {
-    return q4rdna::host::policy_split(rows, cols, cu_count(device), streams, vectors);
+uint32_t policy_split(uint32_t rows, uint32_t cols, int device, bool gate, LaunchKind kind) {
+    return q4rdna::host::policy_split(rows, cols, cu_count(device), gate, kind);
 }
 
-uint32_t resolve_split(const q4rdna_weight *w, uint32_t split, uint32_t streams) {
-    if (split == 0) split = policy_split(w->rows, w->columns, w->device, streams);
+uint32_t resolve_split(const q4rdna_weight *w, uint32_t split, bool gate) {
+    if (split == 0) split = policy_split(w->rows, w->columns, w->device, gate, LaunchKind::kSingle);
     split = std::min(split, w->columns / kGroup);
     split = std::min(split, kMaxSplit);
     return std::max<uint32_t>(split, 1);
@@ -210,7 +211,7 @@ int launch_one(const q4rdna::TensorLaunch &wanted, const q4rdna_weight *w, const
                const float *add, float *y, hipStream_t stream) {
     q4rdna::TensorLaunch launch = wanted;
     if (launch.by_policy && launch.slots > 0 && captured_without_room(w->device, stream, launch.slots)) {
-        launch.split = std::min(policy_split(w->rows, w->columns, w->device, 1, 2), launch.split);
+        launch.split = std::min(policy_split(w->rows, w->columns, w->device, false, LaunchKind::kVectors), launch.split);
         launch.slots = exchange_slots(launch.split, w->rows, gate ? 2 : 1);
     }
     uint32_t *slots = nullptr;
@@ -293,7 +294,7 @@ int check_mul_mat_ex(const q4rdna_weight *w, const q4rdna_weight *gate, const fl
         *launch = L;
         return Q4RDNA_OK;
     }
-    L.split = resolve_split(w, s, gate ? 2 : 1);
+    L.split = resolve_split(w, s, gate != nullptr);
     L.by_policy = s == 0;
     if (!gemv_shape_fits(w->rows / kTileRows, w->columns / kGroup, L.split))
         return set_error(Q4RDNA_ERR_ARGUMENT, "shape %ux%u at split %u is beyond the kernels' index range", w->rows,
@@ -609,7 +610,7 @@ int q4rdna_scope_allows(const char *scope, const char *name) {
 
 uint32_t q4rdna_policy_split_k(uint32_t rows, uint32_t columns, int device) {
     if (!valid_shape(rows, columns)) return 0;
-    return policy_split(rows, columns, device);
+    return policy_split(rows, columns, device, false, LaunchKind::kSingle);
 }
 
 int q4rdna_mul_mat(const q4rdna_weight *w, const float *x, int64_t x_ne0, float *y, int64_t y_ne0, void *stream) {
@@ -683,11 +684,11 @@ int launch_group_valu(const q4rdna_group_desc *descs, uint32_t count, const floa
     if (total_rows > 0x7fffffffull) return set_error(Q4RDNA_ERR_ARGUMENT, "group too large");
     const uint32_t all_rows = static_cast<uint32_t>(total_rows), streams = glu ? 2u : 1u;
     const uint32_t least = (groups + kGroupChunkGroups - 1) / kGroupChunkGroups;
-    uint32_t split = std::max(split_k != 0 ? split_k : policy_split(all_rows, cols, device), least);
-    split = std::min(split, groups);
+    uint32_t split = split_k != 0 ? split_k : policy_split(all_rows, cols, device, glu, LaunchKind::kGroup);
+    split = std::min(std::max(split, least), groups);
     if (split_k == 0 && split > least &&
         captured_without_room(device, stream, exchange_slots(split, all_rows, streams)))
-        split = std::min(split, std::max(policy_split(all_rows, cols, device, 1, 2), least));
+        split = std::min(split, std::max(policy_split(all_rows, cols, device, glu, LaunchKind::kVectors), least));
     if (split > kMaxSplit)
         return set_error(Q4RDNA_NOT_APPLICABLE, "K = %u needs more than %u chunks of %u groups", cols, kMaxSplit,
                          kGroupChunkGroups);
@@ -818,7 +819,7 @@ int q4rdna_mul_mat_batch(const q4rdna_weight *w, const q4rdna_weight *gate, cons
         count_launch(w->tiles, gt, n);
         return Q4RDNA_OK;
     }
-    if (split == 0) split = policy_split(w->rows, w->columns, w->device, 1, n);
+    if (split == 0) split = policy_split(w->rows, w->columns, w->device, gate != nullptr, LaunchKind::kVectors);
     split = std::min(std::max(split, need), std::min(groups, kMaxSplit));
     q4rdna::GemvArgs args{};
     args.w = w->tiles;

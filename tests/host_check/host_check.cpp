@@ -6,8 +6,10 @@
 //
 //   host_check layout            lays out the plans below, checks every
 //                                invariant, prints one JSON line per plan
+//   host_check policy            checks the split policy's table and bounds
 //   host_check inspect FILE...   parses each file as a sidecar image, prints
 //                                one JSON line per file (status, count, error)
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -267,6 +269,67 @@ int run_layout() {
     return g_failures == 0 ? 0 : 1;
 }
 
+// The split policy at 256 CUs: its value on both sides of each of its lines,
+// and bounds that hold for every shape.
+int run_policy() {
+    using q4rdna::host::LaunchKind;
+    using q4rdna::host::policy_split;
+    const LaunchKind single = LaunchKind::kSingle, group = LaunchKind::kGroup, vectors = LaunchKind::kVectors;
+    const struct {
+        uint32_t tiles, groups;
+        bool gate;
+        LaunchKind kind;
+        uint32_t split;
+    } table[] = {
+        // 32 groups per workgroup, up to eight chunks; the shapes of a decoder layer.
+        {128, 64, false, single, 2}, {32, 64, false, single, 2}, {384, 64, false, single, 2}, {384, 64, true, single, 2},
+        {128, 192, false, single, 6}, {64, 448, false, single, 8}, {1, 64, false, single, 4}, {1, 16, false, single, 1},
+        // Six workgroups per CU of these for several vectors, and of chunks longer than 32 groups.
+        {768, 33, false, vectors, 2}, {769, 33, false, vectors, 1}, {192, 257, false, single, 8}, {193, 257, false, single, 7},
+        // 16 groups: from more than one workgroup per CU on, while the fullest CU has no more to do, ...
+        {128, 41, false, single, 2}, {129, 41, false, single, 3}, {341, 41, false, single, 3}, {342, 41, false, single, 2},
+        {384, 41, false, single, 2}, {385, 41, false, single, 3}, {129, 41, false, vectors, 2}, {129, 41, false, group, 3},
+        // ... beyond two chunks with a clear gain there or four per CU, ...
+        {85, 65, false, single, 3}, {86, 65, false, single, 5}, {103, 65, false, single, 3}, {341, 65, false, single, 3},
+        {342, 65, false, single, 5}, {384, 112, false, single, 7}, {384, 112, false, group, 4},
+        // ... and with a gate unless the fullest CU gets an eighth more.
+        {16, 41, true, single, 2}, {24, 41, true, single, 3}, {51, 65, true, single, 5}, {52, 65, true, single, 3},
+        {96, 65, true, single, 5}, {154, 65, true, single, 3},
+        {384, 64, true, single, 2}, {385, 64, true, single, 4}, {385, 64, true, group, 2}, {385, 64, true, vectors, 2},
+        // Tall matrices: up to 32 workgroups per CU, ...
+        {2730, 33, false, single, 3}, {2731, 33, false, single, 1}, {2048, 128, false, single, 4}, {2049, 128, false, single, 1},
+        {2048, 64, true, single, 4}, {2049, 64, true, single, 1}, {1024, 64, true, group, 1},
+        {1024, 64, false, group, 2}, {768, 64, true, group, 2}, {1024, 96, true, group, 3},
+        // ... of chunks that fill their waves where the coarse ones run the pipelined loop.
+        {1024, 65, false, single, 1}, {1024, 67, false, single, 5}, {1024, 65, false, group, 5}, {640, 65, false, single, 5},
+        {400, 193, true, single, 3}, {400, 196, true, single, 7}, {400, 193, false, single, 7}, {400, 193, true, group, 7},
+    };
+    for (const auto &t : table) {
+        const uint32_t got = policy_split(32 * t.tiles, 64 * t.groups, 256, t.gate, t.kind);
+        if (got != t.split)
+            expect(false, ("split " + std::to_string(got) + ", not " + std::to_string(t.split)).c_str(),
+                   std::to_string(t.tiles) + " tiles, " + std::to_string(t.groups) + " groups");
+    }
+    uint64_t most_slots = 0;
+    std::mt19937 rng(7);
+    for (uint32_t i = 0; i < 2000000; ++i) {
+        const uint32_t tiles = 1 + static_cast<uint32_t>(std::exp2(rng() % 17000 / 1000.0));
+        const uint32_t groups = 1 + static_cast<uint32_t>(std::exp2(rng() % 11000 / 1000.0));
+        for (bool gate : {false, true}) {
+            const uint32_t split = policy_split(32 * tiles, 64 * groups, 256, gate, single);
+            const uint32_t coarse = policy_split(32 * tiles, 64 * groups, 256, gate, vectors);
+            expect(split >= coarse && coarse >= 1 && split <= std::min(groups, q4rdna::host::kMaxSplit), "range", "policy");
+            expect(split == 1 || q4rdna::gemv_shape_fits(tiles, groups, split), "index range", "policy");
+            most_slots = std::max<uint64_t>(
+                most_slots, uint64_t(q4rdna::host::exchange_nodes(split)) * 32 * tiles * (gate ? 2 : 1));
+        }
+    }
+    // A policy launch never needs more slots than the no-alloc array holds.
+    expect(most_slots <= Q4RDNA_NOALLOC_SLOTS, "no-alloc slots", "policy");
+    std::printf("{\"most_slots\": %llu, \"failures\": %d}\n", static_cast<unsigned long long>(most_slots), g_failures);
+    return g_failures == 0 ? 0 : 1;
+}
+
 int run_inspect(int argc, char **argv) {
     for (int i = 0; i < argc; ++i) {
         std::ifstream in(argv[i], std::ios::binary);
@@ -375,11 +438,12 @@ int run_tree(MeetsFn meets) {
 int main(int argc, char **argv) {
     if (argc >= 2 && std::strcmp(argv[1], "layout") == 0) return run_layout();
     if (argc >= 2 && std::strcmp(argv[1], "inspect") == 0) return run_inspect(argc - 2, argv + 2);
+    if (argc >= 2 && std::strcmp(argv[1], "policy") == 0) return run_policy();
     if (argc >= 2 && std::strcmp(argv[1], "tree") == 0) return run_tree(real_meets);
     // Planted mistakes in the shape rule: each must be reported as failures.
     if (argc >= 2 && std::strcmp(argv[1], "tree-planted-off-by-one") == 0) return run_tree(planted_off_by_one);
     if (argc >= 2 && std::strcmp(argv[1], "tree-planted-always") == 0) return run_tree(planted_always);
-    std::fprintf(stderr, "usage: host_check layout | inspect FILE... | tree | tree-planted-off-by-one | "
+    std::fprintf(stderr, "usage: host_check layout | policy | inspect FILE... | tree | tree-planted-off-by-one | "
                          "tree-planted-always\n");
     return 2;
 }

@@ -65,7 +65,7 @@ def test_first_call_captured(cuda, rows, cols, gated, warm):
 
 @pytest.mark.parametrize("warm", [False, True])
 @pytest.mark.parametrize("gated", [False, True])
-@pytest.mark.parametrize("heights,cols", [((32 * 385, 32 * 384), 64 * 33), ((16384, 8192, 8192), 64 * 64)])
+@pytest.mark.parametrize("heights,cols", [((32 * 385, 32 * 384), 64 * 33), ((16384, 8192, 8192), 64 * 48)])
 def test_first_group_captured(cuda, heights, cols, gated, warm):
     items = []
     for i, rows in enumerate(heights):

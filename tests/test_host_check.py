@@ -4,7 +4,7 @@ valid, mutated, truncated and random images (statuses against the oracle's
 restatement of the reference loader, source/q4rdna.cu:129-170), and the plan
 layout with its item deal on the Qwen3-8B stacks, batched plans and mixed
 plans (every item dealt exactly once, each workgroup's list ascending,
-scratch regions aligned and disjoint), and the split-K exchange tree's
+scratch regions aligned and disjoint), the split policy, and the split-K exchange tree's
 protocol with the kernels' own shape functions.  CPU only."""
 import json
 import os
@@ -65,6 +65,15 @@ def test_plan_layout_and_deal_under_sanitizers(host_check):
     assert not by["mixed"]["all_per_one"] and by["mixed"]["both_streams"]
     assert by["mixed_small_gpu"]["workgroups"] == 16
     assert by["one_gemv"]["items"] == 1
+
+
+def test_split_policy(host_check):
+    """The split on both sides of each line of the policy, its range over two
+    million shapes, and that no policy launch needs more exchange slots than
+    the no-alloc array holds."""
+    r, lines = run(host_check, "policy")
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr
+    assert lines[-1]["failures"] == 0 and 0 < lines[-1]["most_slots"] <= 1 << 21
 
 
 def test_sidecar_parser_under_sanitizers(host_check, golden, tmp_path):
