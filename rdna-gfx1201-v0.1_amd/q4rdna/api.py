@@ -26,7 +26,12 @@ def packed_size(rows: int, cols: int) -> int:
 # torch's current stream of a device index as a handle, without the Stream
 # object that torch.cuda.current_stream builds around it: 0.08 us against
 # 2.0 us, in a call whose kernel takes four.
-_raw_stream = torch._C._cuda_getCurrentRawStream
+try:
+    _raw_stream = torch._C._cuda_getCurrentRawStream
+except AttributeError:  # a torch build without this private function
+
+    def _raw_stream(device: int) -> int:
+        return torch.cuda.current_stream(device).cuda_stream
 
 
 def _stream(device: torch.device | int | None = None) -> int:
