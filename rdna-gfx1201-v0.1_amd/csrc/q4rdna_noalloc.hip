@@ -22,7 +22,6 @@
 #include <mutex>
 
 #include "q4rdna.h"
-#include "q4rdna_host.h"
 #include "q4rdna_internal.h"
 #include "q4rdna_runtime.h"
 
@@ -68,14 +67,6 @@ extern "C" int q4rdna_mul_mat_ex_noalloc(const q4rdna_weight *w, const q4rdna_we
     if (rc != Q4RDNA_OK) return rc;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const uint8_t *gt = gate ? gate->tiles : nullptr;
-    // The policy's split is a choice: a tall matrix whose chunks would need
-    // more slots than there are takes fewer.
-    if (L.by_policy) {
-        while (L.slots > Q4RDNA_NOALLOC_SLOTS) {
-            L.split /= 2;
-            L.slots = L.split < 2 ? 0 : static_cast<size_t>(q4rdna::host::exchange_nodes(L.split)) * w->rows * (gate ? 2 : 1);
-        }
-    }
     if (L.slots == 0) {
         if ((rc = q4rdna::launch_tensor_in(L, w, gt, x, add, y, nullptr, s)) == Q4RDNA_OK)
             q4rdna::count_gemv_launch(w->tiles, gt);
