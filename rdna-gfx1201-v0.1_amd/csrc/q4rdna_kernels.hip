@@ -952,7 +952,9 @@ __device__ uint32_t search_experiment(const float *v, const GroupRange &g, int a
 // Thread per (row, group) ordered (row tile, group, row lane) so a wave's
 // scale and code stores land in contiguous bytes of one tile.  Bound by the
 // search's arithmetic, ten VALU operations per value and evaluation:
-// 12288x4096 takes 836 us, with a division per value and evaluation and the
+// 12288x4096 takes 836 us, and took 6257 with a division per value and
+// evaluation and the wave in step over the starts.  The sidecar search runs in
+// 104 VGPRs, four waves per SIMD (its 32 KB of LDS leaves five).
 template <bool SIDECAR>
 __global__ __launch_bounds__(kThreads, SIDECAR ? 3 : 1) void pack_kernel(const float *__restrict__ w, uint32_t rows,
                                                                          uint32_t cols, int algorithm,
