@@ -127,10 +127,10 @@ int q4rdna_scope_allows(const char *scope, const char *name);
  * Launches with split K use a scratch buffer per (device, stream).  The
  * first call that needs more than the stream has allocates it, which it
  * cannot do while that stream is being captured (other streams may be): make
- * one call of each shape on the stream before capturing.  (A policy-chosen split of
- * a tall matrix or group, captured without that call, takes fewer chunks
- * instead, so another order of each row's sum and other last bits than the
- * eager call's; it is refused only where these need a larger buffer too.)
+ * one call of each shape on the stream before capturing.  (A policy-chosen
+ * split of a tall matrix or group, captured without that call, takes fewer
+ * chunks instead, so another order of each row's sum and other last bits than
+ * the eager call's; it is refused only where these need a larger buffer too.)
  * Outgrown buffers are never freed, so a graph captured earlier stays
  * valid.  Calls on one stream are ordered by it; a graph must not replay on
  * another stream while the stream it was captured on runs such calls.
